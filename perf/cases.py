@@ -1,0 +1,450 @@
+"""Measured workloads of the renderer: what its users have it do, through lambda_amd.gpu and
+lambda_amd.diff, with inputs made from a seed.
+
+A case is a dict of plain values. Its "kind" names the call, the rest are sizes and options:
+
+  render   a film rendered from nothing and read back (gpu.render): "scene" is one of cornell,
+           nodes (Cornell room with procedural shader networks), instanced, many_light, media (density
+           grid in a pass-through box) and fog (homogeneous medium in the Cornell room)
+  guided   one wave of a render guided by a trained network (render_desc(guide=...))
+  batch    many small scenes in one call (gpu.render_batch)
+  inverse  one optimisation step of a differentiable render, forward and backward (diff.DiffRenderer)
+  train    one gradient of the guiding network over a batch of records (Guide.gradient)
+  image    denoise, tone map and 8-bit packing of a rendered film (Film.denoise, Film.post)
+  rays     closest hits and occlusion of a caller's own rays (Scene.intersect, Scene.occluded)
+"""
+import math
+
+import numpy as np
+import torch
+
+from lambda_amd import abi, diff, gpu, scene
+
+_DEVICE = None
+
+INTEGRATORS = {"path": abi.INTEGRATOR_PATH, "direct": abi.INTEGRATOR_DIRECT, "volpath": abi.INTEGRATOR_VOLPATH,
+               "mis_volpath": abi.INTEGRATOR_MIS_VOLPATH, "normal": abi.INTEGRATOR_NORMAL}
+
+
+def _device():
+    """One device handle per program, as a renderer holds it (it owns the path pool)."""
+    global _DEVICE
+    if _DEVICE is None:
+        _DEVICE = gpu.Device(0)
+    return _DEVICE
+
+
+def _render(name, sc, w, h, spp, depth, integrator="path", spectral="hero4", estimator="corrected", lights="tree", size=0):
+    return dict(name=name, kind="render", scene=sc, w=w, h=h, spp=spp, depth=depth, integrator=integrator,
+                spectral=spectral, estimator=estimator, lights=lights, size=size)
+
+
+def listed():
+    return [
+        # one pass of an interactive preview: the smallest call a viewer makes, again and again
+        _render("preview_cornell_64", "cornell", 64, 64, 1, 8),
+        # the Cornell box at its usual size, a final render of a small scene
+        _render("cornell_256_64spp", "cornell", 256, 256, 64, 8),
+        # the headline workload: 1.2M triangles, 4,096 emissive triangles, sky, thin lens, 1080p
+        _render("many_light_1080p_32spp", "many_light", 1920, 1080, 32, 16, size=200),
+        # the reference-compatible estimator in RGB with the power light sampler, a ragged size, shader networks
+        _render("nodes_faithful_517x389", "nodes", 517, 389, 6, 8, spectral="rgb", estimator="faithful", lights="power"),
+        # the heterogeneous-media workload: 128^3 density grid, 65 lights, MIS volumetric integrator
+        _render("media_1024_4spp", "media", 1024, 1024, 4, 32, integrator="mis_volpath", size=128),
+        # plain volumetric path tracing in RGB through a homogeneous fog, ragged size
+        _render("fog_301x211_16spp", "fog", 301, 211, 16, 12, integrator="volpath", spectral="rgb"),
+        # a guided wave after training: network inference between extension and shading
+        dict(name="guided_960x540_8spp", kind="guided", w=960, h=540, spp=8, depth=16, size=60),
+        # a parameter sweep or data set: small scenes of different sizes rendered in one call
+        dict(name="batch_8_scenes", kind="batch", jobs=8, spp=2, largest=384),
+        # inverse rendering: loss gradient of two textures and a density grid
+        dict(name="inverse_512_8spp", kind="inverse", w=512, h=512, spp=8, tex=512, grid=64),
+        # one training gradient of the guiding network at its default batch
+        dict(name="train_16384_records", kind="train", records=16384),
+        # the last steps of a frame: denoise with normal and albedo guides, ACES, gamma, 8 bits
+        dict(name="image_1080p", kind="image", w=1920, h=1080, iterations=5),
+        # ray queries against a mesh: a baker's or a collision test's batch
+        dict(name="rays_1m", kind="rays", rays=1000003, size=60),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    """One more case of the same ranges."""
+    kind = rng.choice(["render"] * 6 + ["guided", "batch", "inverse", "train", "image", "rays"])
+    if kind == "render":
+        sc = rng.choice(["cornell", "nodes", "instanced", "many_light", "many_light", "media", "fog"])
+        volume = sc in ("media", "fog")
+        w, h = _log(rng, 24, 1280), _log(rng, 24, 1024)
+        spp = max(1, min(_log(rng, 1, 64), (4 << 20) // (w * h) if volume else (16 << 20) // (w * h)))
+        integ = rng.choice(["volpath", "mis_volpath"]) if volume else rng.choice(["path"] * 5 + ["direct", "normal"])
+        only_corrected = integ == "normal" or sc == "media"  # as written these passes are black or tinted
+        return dict(kind=kind, scene=sc, w=w, h=h, spp=spp, depth=rng.choice([6, 8, 12, 16]), integrator=integ,
+                    spectral=rng.choice(["hero4", "rgb"]),
+                    estimator="corrected" if only_corrected else rng.choice(["corrected", "corrected", "faithful"]),
+                    lights=rng.choice(["tree", "tree", "power"]),
+                    size=_log(rng, 4, 80) if sc == "many_light" else (rng.randint(24, 128) if sc == "media" else 0))
+    if kind == "guided":
+        w, h = _log(rng, 48, 960), _log(rng, 48, 640)
+        return dict(kind=kind, w=w, h=h, spp=max(1, min(_log(rng, 1, 32), (4 << 20) // (w * h))), depth=rng.choice([8, 16]),
+                    size=_log(rng, 4, 60))
+    if kind == "batch":
+        return dict(kind=kind, jobs=rng.randint(2, 8), spp=rng.randint(1, 3), largest=_log(rng, 48, 384))
+    if kind == "inverse":
+        w, h = _log(rng, 32, 512), _log(rng, 32, 512)
+        return dict(kind=kind, w=w, h=h, spp=max(1, min(_log(rng, 2, 32), (2 << 20) // (w * h))), tex=_log(rng, 32, 512),
+                    grid=rng.randint(16, 64))
+    if kind == "train":
+        return dict(kind=kind, records=_log(rng, 64, 65536))
+    if kind == "image":
+        return dict(kind=kind, w=_log(rng, 64, 1920), h=_log(rng, 48, 1080), iterations=rng.randint(1, 6))
+    return dict(kind=kind, rays=_log(rng, 1000, 1500000), size=_log(rng, 4, 60))
+
+
+# ---------------------------------------------------------------- inputs
+def _cloud(seed, res):
+    """A res^3 density grid like the fBm clouds of the media workloads: five octaves of smooth
+    noise, clipped at zero."""
+    g = torch.Generator().manual_seed(seed)
+    acc = torch.zeros(1, 1, res, res, res)
+    for o in range(5):
+        n = min(res, 4 << o)
+        acc += 0.5 ** o * torch.nn.functional.interpolate(torch.rand(1, 1, n, n, n, generator=g) * 2 - 1, size=(res,) * 3,
+                                                          mode="trilinear", align_corners=False)
+    return np.ascontiguousarray(acc.clamp_min(0)[0, 0].numpy())
+
+
+def _media_scene(seed, res):
+    """The media workload's layout: a density grid in [-1, 1]^3, a spotlight above, 64 point lights around."""
+    sd = scene.SceneDesc()
+    med = scene.grid_medium(sd, _cloud(seed, res), [0.4] * 3, [3.6] * 3, 0.6, (-1.0, -1.0, -1.0), (1.0, 1.0, 1.0))
+    box = sd.add_material(scene.passthrough(interior=med))
+    v, i = scene.aabb((-1.0, -1.0, -1.0), (1.0, 1.0, 1.0))
+    sd.add_mesh(v, i, box)
+    sd.add_spot_light((0.0, 3.0, 0.0), (0.0, -1.0, 0.0), math.radians(30.0), math.radians(20.0), 30.0, temperature=5000.0)
+    golden = math.pi * (3.0 - math.sqrt(5.0))
+    for k in range(64):
+        y = 1.0 - 2.0 * (k + 0.5) / 64
+        r = math.sqrt(max(0.0, 1.0 - y * y))
+        sd.add_point_light((3.0 * r * math.cos(golden * k), 3.0 * y, 3.0 * r * math.sin(golden * k)), 1.5,
+                           temperature=3000.0 + 6000.0 * (k % 8) / 7.0)
+    return sd
+
+
+def _many_light(size, seed):
+    """A part of the many-light field: `size` spheres of 5,120 triangles, ground, quads and sky in proportion."""
+    return scene.many_light_scene(n_spheres=size, sphere_level=4, ground_res=max(16, int(297 * math.sqrt(size / 200))),
+                                  n_light_quads=max(8, 2048 * size // 200), seed=seed % (1 << 20))
+
+
+def _scene(case, seed):
+    """(SceneDesc, camera) of a render case."""
+    w, h, name = case["w"], case["h"], case["scene"]
+    if name == "many_light":
+        return _many_light(case["size"], seed), scene.many_light_camera(w, h)
+    if name == "media":
+        return _media_scene(seed, case["size"]), scene.media_camera(w, h)
+    if name == "cornell":
+        return scene.cornell_box(temperature=4000.0 + seed % 3000), scene.cornell_camera(w, h)
+    if name == "nodes":
+        return scene.procedural_cornell(), scene.cornell_camera(w, h)
+    if name == "instanced":
+        return scene.instanced_cornell(seed=seed % (1 << 20)), scene.cornell_camera(w, h)
+    return scene.fog_cornell(sigma_scale=0.75 + (seed % 101) / 200.0), scene.cornell_camera(w, h)
+
+
+def _push(sd, lights="tree"):
+    s = gpu.Scene(_device())
+    sd.push(s, abi.LIGHTS_TREE if lights == "tree" else abi.LIGHTS_POWER)
+    return s
+
+
+def _bf16(a):
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to(torch.bfloat16).float().numpy()
+
+
+GUIDE_SHAPES = [(64, 80)] + [(64, 64)] * 4 + [(144, 64)]
+
+
+def _guide_params(seed):
+    """A network like a trained one: He-uniform hidden layers, a modest output layer, BF16 weights."""
+    rng = np.random.default_rng(seed)
+    w = [_bf16(rng.uniform(-1, 1, r * c) * math.sqrt(6.0 / c) * (0.3 if r == 144 else 1.0)) for r, c in GUIDE_SHAPES]
+    b = [rng.uniform(-0.1, 0.1, r).astype(np.float32) for r, _ in GUIDE_SHAPES]
+    return np.concatenate(w + b)
+
+
+def _records(n, seed):
+    rng = np.random.default_rng(seed + 1)
+    r = np.zeros((n, 8), dtype=np.float32)
+    r[:, :5] = rng.uniform(0, 1, size=(n, 5))
+    r[:, 5] = rng.integers(0, 128, size=n)
+    r[:, 6] = rng.uniform(0.01, 2.0, size=n)
+    r[:, 7] = rng.exponential(1.0, size=n)
+    r[::7, 7] = 0.0  # records that carried no radiance
+    return r
+
+
+def _frame(w, h, seed):
+    """(colour, albedo, normal) as a low-sample render gives them, float32 values: noisy radiance over
+    blocks of materials, albedo and normals constant in each block."""
+    g = torch.Generator().manual_seed(seed)
+    gh, gw = max(1, -(-h // 37)), max(1, -(-w // 53))
+
+    def blocks(lo, hi):
+        c = torch.rand(gh, gw, 3, generator=g) * (hi - lo) + lo
+        return c.repeat_interleave(37, 0)[:h].repeat_interleave(53, 1)[:, :w]
+    albedo = blocks(0.05, 0.95)
+    normal = blocks(0.0, 1.0)
+    light = 0.4 + blocks(0.0, 1.2)
+    noise = -torch.log(torch.rand(h, w, 3, generator=g).clamp_min(1e-6))  # exponential, mean 1
+    colour = albedo * light * noise
+    return [np.ascontiguousarray(t.float().double().numpy()) for t in (colour, albedo, normal)]
+
+
+def _batch_job(k, jobs, largest, seed):
+    """Job k of a batch: scenes of 1 to 12 spheres and images from 40 pixels to `largest`, one in four with a cloud."""
+    rng = np.random.default_rng(1000 * seed + k)
+    media = k % 4 == 3
+    sd = scene.many_light_scene(n_spheres=int(rng.integers(1, 13)), sphere_level=3, ground_res=int(rng.integers(8, 64)),
+                                n_light_quads=int(rng.integers(8, 128)), env=not media, seed=int(rng.integers(1 << 20)))
+    if media:
+        med = scene.grid_medium(sd, _cloud(int(rng.integers(1 << 30)), 32), (0.3, 0.3, 0.3), (1.2, 1.1, 1.0), 0.4,
+                                (-20.0, 1.5, -20.0), (20.0, 4.0, 20.0))
+        fog = sd.add_material(scene.passthrough(interior=med))
+        v, i = scene.aabb((-20.0, 1.5, -20.0), (20.0, 4.0, 20.0))
+        sd.add_mesh(v, i, fog)
+    side = max(40, largest * (k + 1) // jobs)
+    return sd, scene.many_light_camera(side, side), side, abi.INTEGRATOR_VOLPATH if media else abi.INTEGRATOR_PATH
+
+
+def _film_desc(case, s, cam, film, seed):
+    return gpu.render_desc(s, film, cam, 0, case["spp"], max_bounces=case["depth"], min_bounces=3,
+                           spectral=abi.SPECTRAL_HERO4 if case["spectral"] == "hero4" else abi.SPECTRAL_RGB,
+                           estimator=abi.ESTIMATOR_CORRECTED if case["estimator"] == "corrected" else abi.ESTIMATOR_FAITHFUL,
+                           seed=seed & 0xFFFFFFFF, integrator=INTEGRATORS[case["integrator"]])
+
+
+def prepare(case, seed):
+    """What a program holds before the call: committed scenes, films, the network, host rays or parameter tensors."""
+    kind = case["kind"]
+    if kind == "render":
+        sd, cam = _scene(case, seed)
+        s = _push(sd, case["lights"])
+        film = gpu.Film(_device(), case["w"], case["h"])
+        return dict(kind=kind, case=case, scene=s, film=film, desc=_film_desc(case, s, cam, film, seed))
+    if kind == "guided":
+        s = _push(_many_light(case["size"], seed))
+        film = gpu.Film(_device(), case["w"], case["h"])
+        guide = gpu.Guide(_device(), seed=seed & 0xFFFF, max_depth=2)
+        guide.set_params(_guide_params(seed))
+        d = gpu.render_desc(s, film, scene.many_light_camera(case["w"], case["h"]), 0, case["spp"],
+                            max_bounces=case["depth"], min_bounces=3, spectral=abi.SPECTRAL_HERO4,
+                            estimator=abi.ESTIMATOR_CORRECTED, seed=seed & 0xFFFFFFFF, guide=guide)
+        return dict(kind=kind, case=case, scene=s, film=film, guide=guide, desc=d)
+    if kind == "batch":
+        scenes, films, descs = [], [], []
+        for k in range(case["jobs"]):
+            sd, cam, side, integ = _batch_job(k, case["jobs"], case["largest"], seed % (1 << 20))
+            s = _push(sd)
+            f = gpu.Film(_device(), side, side)
+            scenes.append(s)
+            films.append(f)
+            descs.append(gpu.render_desc(s, f, cam, 0, case["spp"], max_bounces=8, min_bounces=3,
+                                         spectral=abi.SPECTRAL_HERO4, estimator=abi.ESTIMATOR_CORRECTED,
+                                         seed=seed & 0xFFFFFFFF, integrator=integ))
+        return dict(kind=kind, case=case, scenes=scenes, films=films, descs=descs)
+    if kind == "inverse":
+        rng = np.random.default_rng(seed)
+        t, g = case["tex"], case["grid"]
+        alb = scene._smooth_field(rng, t, 16, 0.25, 0.85, 3)
+        rough = scene._smooth_field(rng, t, 16, 0.2, 0.7)
+        dens = _cloud(seed, g) * 1.5
+        sd, ids = scene.inverse_scene(tex_res=t, grid_res=g, seed=seed % (1 << 20), albedo=alb, roughness=rough, density=dens)
+        r = diff.DiffRenderer(_device(), sd, scene.inverse_camera(case["w"], case["h"]), case["w"], case["h"], case["spp"],
+                              [("texture", ids["albedo"]), ("texture", ids["roughness"]), ("density", ids["medium"])])
+        params = [torch.from_numpy(np.ascontiguousarray(p, dtype=np.float32)).cuda().requires_grad_()
+                  for p in (alb, rough, dens)]
+        target = torch.full((case["h"], case["w"], 3), 0.5, device="cuda")
+        return dict(kind=kind, case=case, renderer=r, params=params, target=target, seed=seed & 0xFFFFFF)
+    if kind == "train":
+        guide = gpu.Guide(_device(), seed=seed & 0xFFFF, record_capacity=1 << 16)
+        guide.set_params(_guide_params(seed))
+        return dict(kind=kind, case=case, guide=guide, records=_records(case["records"], seed))
+    if kind == "image":
+        films = []
+        for a in _frame(case["w"], case["h"], seed):
+            f = gpu.Film(_device(), case["w"], case["h"])
+            f.write(a)
+            films.append(f)
+        out = gpu.Film(_device(), case["w"], case["h"])
+        dn = abi.denoise_desc(iterations=case["iterations"], sigma_colour=0.8, sigma_normal=0.2, sigma_albedo=0.1)
+        post, _ = abi.post_desc()
+        return dict(kind=kind, case=case, films=films, out=out, denoise=dn, post=post)
+    s = _push(_many_light(case["size"], seed))
+    rng = np.random.default_rng(seed)
+    n = case["rays"]
+    o = rng.uniform((-20.0, 0.05, -20.0), (20.0, 4.0, 20.0), size=(n, 3))
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    tmax = np.full((n, 1), np.inf)
+    rays = np.ascontiguousarray(np.concatenate([o, np.zeros((n, 1)), d, tmax], axis=1), dtype=np.float32)
+    return dict(kind=kind, case=case, scene=s, rays=rays)
+
+
+def run(state):
+    kind = state["kind"]
+    if kind in ("render", "guided"):
+        film = state["film"]
+        film.clear()
+        gpu.render(state["desc"])
+        if kind == "render" and state["case"]["spp"] == 1:
+            return film.read_rgba()  # what a viewer shows
+        return list(film.read())
+    if kind == "batch":
+        for f in state["films"]:
+            f.clear()
+        gpu.render_batch(state["descs"])
+        return [f.read_rgba() for f in state["films"]]
+    if kind == "inverse":
+        img = state["renderer"].render(*state["params"], seed=state["seed"])
+        loss = ((img - state["target"]) ** 2).mean()
+        grads = torch.autograd.grad(loss, state["params"])
+        return dict(image=img, albedo=grads[0], roughness=grads[1], density=grads[2])
+    if kind == "train":
+        g, loss = state["guide"].gradient(state["records"])
+        return dict(grad=g, loss=loss)
+    if kind == "image":
+        colour, albedo, normal = state["films"]
+        colour.denoise(state["denoise"], albedo=albedo, normal=normal, out=state["out"])
+        f32, u8 = state["out"].post(state["post"])
+        return dict(f32=f32, u8=u8)
+    hits = state["scene"].intersect(state["rays"])
+    occ = state["scene"].occluded(state["rays"])
+    return dict(tuv=hits[:, :3].view(np.float32), prim=hits[:, 3].view(np.int32), occluded=occ.view(np.int32))
+
+
+# ---------------------------------------------------------------- what a pass needs, and how close two passes are
+# Path vertices per sample (measured with the traversal counters), and the arithmetic of one vertex: about
+# twenty 4-wide box tests of 60 operations, three triangle tests of 40 and some 600 of shading.
+VERTICES = {"cornell": 4.0, "nodes": 4.0, "instanced": 4.0, "many_light": 2.2, "media": 9.0, "fog": 7.0}
+VERTEX_FLOPS = 2000.0
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("render", "guided", "inverse"):
+        px = case["w"] * case["h"]
+        sc = case.get("scene", "many_light")
+        per = 1.0 if case.get("integrator") in ("direct", "normal") else VERTICES[sc]
+        flops = px * case["spp"] * per * VERTEX_FLOPS
+        size = case.get("size", 9)
+        tris = 6000 * size if sc == "many_light" else 5000
+        byt = 28.0 * px + 48.0 * tris + (4.0 * size ** 3 if sc == "media" else 0.0)
+        if kind == "guided":
+            flops += 61440.0 * 2 * px * case["spp"]  # the network at the first two vertices
+        if kind == "inverse":
+            flops *= 3.0  # the loss's forward render, then the primal pass and its replay
+            byt = 2 * (28.0 * px + 48.0 * 50688) + 2 * (16.0 * case["tex"] ** 2 + 4.0 * case["grid"] ** 3)
+        return dict(bytes=byt, flops=flops)
+    if kind == "batch":
+        px = sum(max(40, case["largest"] * (k + 1) // case["jobs"]) ** 2 for k in range(case["jobs"]))
+        return dict(bytes=16.0 * px + 48.0 * 20000 * case["jobs"], flops=px * case["spp"] * 2.5 * VERTEX_FLOPS)
+    if kind == "train":
+        n = case["records"]
+        return dict(bytes=32.0 * n + 8.0 * 31184, flops=3 * 61440.0 * n)
+    if kind == "image":
+        px = case["w"] * case["h"]  # three films in; 25 taps of 20 operations per pass; the film, 16 + 4 B out
+        return dict(bytes=px * (3 * 28.0 + 28.0 + 20.0), flops=px * (case["iterations"] * 25 * 24.0 + 100.0))
+    n = case["rays"]
+    return dict(bytes=32.0 * n + 20.0 * n + 48.0 * 6000 * case["size"], flops=2 * n * 1300.0)
+
+
+def tolerance(case):
+    kind = case["kind"]
+    if kind == "rays":
+        return "exact"  # the closest hit is defined bit for bit: ties go to the smaller primitive
+    if kind == "image":
+        return {"rel": 5e-7, "max": 2e-5, "differ": 1e-4}  # 8.4e-8 from 64 bits; 8-bit roundings
+    if kind == "train":
+        return {"rel": 4e-3}  # BF16 activations through six layers: 1.0e-3 from 64 bits
+    # A difference in a last bit (a library's exp, another order) sends up to one path in a thousand
+    # another way. Films of 192 x 108 pixels against a CPU implementation of the same estimator, with
+    # another mathematics library: up to 9e-4 of the paths differ, rel 3e-7 to 2.6e-3 and max up to 0.31
+    # (one bright path) on the many-light field, rel 3.6e-4 and max 0.02 on the media.
+    return {"rel": 0.01, "max": 0.999}
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind == "train":
+        return _exact_gradient(_guide_params(seed), _records(case["records"], seed))
+    if kind == "image":
+        return dict(f32=_exact_image(case, seed), u8=None)
+    return None
+
+
+def _exact_gradient(p, rec):
+    """Loss and gradient of the guiding objective in 64 bits, by autograd."""
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    flat = torch.from_numpy(p).to(dev, torch.float64).requires_grad_()
+    r = torch.from_numpy(rec).to(dev, torch.float64)
+    o = torch.arange(8, device=dev, dtype=torch.float64)
+    t = torch.frac(r[:, :5, None] * 2.0 ** (o - 1)) * (2 * math.pi)  # octaves of each input
+    x = torch.stack([torch.sin(t), torch.cos(t)], -1).reshape(len(r), 80)
+    w_off, b_off = 0, sum(a * b for a, b in GUIDE_SHAPES)
+    for k, (rows, cols) in enumerate(GUIDE_SHAPES):
+        w = flat[w_off:w_off + rows * cols].reshape(rows, cols)
+        x = x @ w.t() + flat[b_off:b_off + rows]
+        if k < len(GUIDE_SHAPES) - 1:
+            x = torch.relu(x)
+        w_off += rows * cols
+        b_off += rows
+    q = torch.softmax(x[:, :128], 1).gather(1, r[:, 5:6].long())[:, 0] / (4 * math.pi / 128)
+    c = 0.05 + 0.85 * torch.sigmoid(x[:, 128])
+    wt = r[:, 7] / r[:, 7].sum()
+    loss = -(wt * torch.log(c * q + (1 - c) * r[:, 6])).sum()
+    grad, = torch.autograd.grad(loss, flat)
+    return dict(grad=grad, loss=float(loss))
+
+
+def _exact_image(case, seed):
+    """Edge-avoiding A-Trous filter, fitted ACES and clamp in 64 bits (alpha 1)."""
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    colour, albedo, normal = (torch.from_numpy(a).to(dev) for a in _frame(case["w"], case["h"], seed))
+    h, w = case["h"], case["w"]
+    div = torch.where(albedo > float(np.float32(1e-3)), albedo, torch.ones_like(albedo))
+    c = colour / div
+    kern = (0.0625, 0.25, 0.375, 0.25, 0.0625)
+    for i in range(case["iterations"]):
+        step, sc = 1 << i, 0.8 * 0.5 ** i
+        acc, tot = torch.zeros_like(c), torch.zeros(h, w, 1, device=dev, dtype=torch.float64)
+        for dy in range(-2, 3):
+            ya, yb = max(0, -dy * step), min(h, h - dy * step)
+            if ya >= yb:
+                continue
+            for dx in range(-2, 3):
+                xa, xb = max(0, -dx * step), min(w, w - dx * step)
+                if xa >= xb:
+                    continue
+                here = (slice(ya, yb), slice(xa, xb))
+                there = (slice(ya + dy * step, yb + dy * step), slice(xa + dx * step, xb + dx * step))
+                e = ((c[there] - c[here]) ** 2).sum(-1, keepdim=True) / sc ** 2
+                e = e + ((normal[there] - normal[here]) ** 2).sum(-1, keepdim=True) / 0.2 ** 2
+                e = e + ((albedo[there] - albedo[here]) ** 2).sum(-1, keepdim=True) / 0.1 ** 2
+                wt = kern[dy + 2] * kern[dx + 2] * torch.exp(-e)
+                acc[here] += wt * c[there]
+                tot[here] += wt
+        c = acc / tot
+    c = c * div
+    m_in = torch.tensor([[0.59719, 0.35458, 0.04823], [0.07600, 0.90834, 0.01566], [0.02840, 0.13383, 0.83777]],
+                        device=dev, dtype=torch.float64)
+    m_out = torch.tensor([[1.60475, -0.53108, -0.07367], [-0.10208, 1.10813, -0.00605], [-0.00327, -0.07276, 1.07602]],
+                         device=dev, dtype=torch.float64)
+    v = c @ m_in.t()
+    v = (v * (v + 0.0245786) - 0.000090537) / (v * (0.983729 * v + 0.4329510) + 0.238081)
+    v = (v @ m_out.t()).clamp(0.0, 1.0)
+    return torch.cat([v, torch.ones(h, w, 1, device=dev, dtype=torch.float64)], -1)
