@@ -27,10 +27,16 @@ INTEGRATORS = {"path": abi.INTEGRATOR_PATH, "direct": abi.INTEGRATOR_DIRECT, "vo
 
 
 def _device():
-    """One device handle per program, as a renderer holds it (it owns the path pool)."""
+    """One device handle per program, as a renderer holds it. A start-up render with an explicit path
+    capacity sizes the path pool that the handle keeps, so that no later render has to grow it."""
     global _DEVICE
     if _DEVICE is None:
         _DEVICE = gpu.Device(0)
+        s = _push(_many_light(200, 0))
+        film = gpu.Film(_DEVICE, 16, 16)
+        gpu.render(gpu.render_desc(s, film, scene.many_light_camera(16, 16), 0, 1, capacity=1 << 27))
+        film.close()
+        s.close()
     return _DEVICE
 
 
