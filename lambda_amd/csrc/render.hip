@@ -846,7 +846,10 @@ struct Wave {
     return b;
   }
   lgpu_status alloc(uint32_t n, uint32_t spillWords, bool guided = false) {
+    // also for n <= cap: a scene with a deeper tree needs more words per path, and growing the spill
+    // area moves it
     LGPU_HIP(spill.alloc(std::max<size_t>(256, 4ull * spillWords * n)));
+    spill_p = spill.as<uint32_t>();
     if (guided) {
       LGPU_HIP(gbins.alloc(128ull * n));
       LGPU_HIP(ghdr.alloc(8ull * n));
@@ -860,6 +863,7 @@ struct Wave {
         for (hipEvent_t &e : row) LGPU_HIP(hipEventCreate(&e));
     }
     if (n <= cap) return LGPU_OK;
+    cap = 0;  // until every part has grown: a failed growth leaves parts released
     for (int b = 0; b < 2; ++b) {
       for (int k = 0; k < 9; ++k) LGPU_HIP(st[b][k].alloc(16ull * n));
       PathState &p = ps[b];
@@ -871,7 +875,7 @@ struct Wave {
     LGPU_HIP(shadow.alloc(sizeof(ShadowRay) * (size_t)n));
     LGPU_HIP(counters.alloc(64)); LGPU_HIP(tcount.alloc(64)); LGPU_HIP(scene.alloc(sizeof(DevScene)));
     ss.L = L.as<float4>(); ss.pixel = pix.as<uint32_t>(); ss.lambda0 = lam.as<float>();
-    shadow_p = shadow.as<ShadowRay>(); counters_p = counters.as<uint32_t>(); spill_p = spill.as<uint32_t>();
+    shadow_p = shadow.as<ShadowRay>(); counters_p = counters.as<uint32_t>();
     tcount_p = tcount.as<unsigned long long>(); scene_p = scene.as<DevScene>();
     cap = n;
     return LGPU_OK;
