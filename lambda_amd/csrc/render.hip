@@ -17,6 +17,7 @@
 #include "guide.h"
 #include "host.h"
 #include "lights.h"
+#include "queue.h"
 #include "shading.h"
 #include "trace.h"
 
@@ -242,14 +243,8 @@ __device__ inline void PushShadow(const Queues &q, const ShadowSpec &sh, uint32_
   q.shadow[slot] = r;
 }
 
-// Queue slots are handed out per block: a device-scope atomic on one counter serialises across
-// the whole GPU (about 11 ns each on MI355X, measured), so one per block and queue instead of one
-// per wave cuts that cost fourfold. The block's pushes are collected (the extension ray in
-// registers, the shadow ray staged in LDS) and written after one allocation at the block's end.
-struct ExtPush {
-  float4 o, d, beta, mis, pp, pn;
-  uint4 ids, aux;
-};
+// The path shade stage's pushes: the extension ray in registers (ExtPush), the shadow ray staged in
+// LDS, both written after one allocation at the block's end (queue.h).
 __device__ inline void StageShadow(ShadowRay &r, const ShadowSpec &sh, uint32_t sid, Spec c) {
   r.o[0] = sh.o.x; r.o[1] = sh.o.y; r.o[2] = sh.o.z; r.tmax = sh.tmax;
   r.d[0] = sh.d.x; r.d[1] = sh.d.y; r.d[2] = sh.d.z; r.sid = sid;
@@ -289,14 +284,7 @@ __device__ inline void BlockPush(const Queues &q, bool pushE, const ExtPush &e, 
   const uint64_t below = (1ull << lane) - 1ull;
   if (pushE) {
     const uint32_t j = bases[0] + cnt[0][wv] + (uint32_t)__popcll(mE & below);
-    q.next.ray_o[j] = e.o;
-    q.next.ray_d[j] = e.d;
-    q.next.beta[j] = e.beta;
-    q.next.ids[j] = e.ids;
-    q.next.aux[j] = e.aux;
-    q.next.mis[j] = e.mis;
-    q.next.prev_p[j] = e.pp;
-    q.next.prev_n[j] = e.pn;
+    WriteExt(q.next, j, e);
   }
   if (pushS) q.shadow[bases[1] + cnt[1][wv] + (uint32_t)__popcll(mS & below)] = stage[threadIdx.x];
 }

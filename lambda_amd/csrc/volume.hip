@@ -17,6 +17,7 @@
 #include "host.h"
 #include "lights.h"
 #include "media.h"
+#include "queue.h"
 #include "shading.h"
 #include "trace.h"
 
@@ -34,16 +35,17 @@ struct PathOut {  // continuation written to the next queue
   bool medInter = false;  // the vertex is a medium interaction (its deferred light lookup reads 3-D textures)
 };
 
-__device__ inline void Push(const Queues &q, const uint4 &ids, uint32_t sid, uint32_t dim, float l0, const PathOut &p) {
-  const uint32_t j = atomicAdd(&q.counters[0], 1u);
-  q.next.ray_o[j] = ToF4(p.o, l0);
-  q.next.ray_d[j] = ToF4(p.d, p.eta);
-  q.next.beta[j] = F4(p.beta);
-  q.next.ids[j] = make_uint4(ids.x, ids.y, dim, (p.depth << 8) | p.flags);
-  q.next.aux[j] = make_uint4(sid, p.pick, p.pass, p.med);
-  q.next.mis[j] = p.mis;
-  q.next.prev_p[j] = ToF4(p.prevP, 0.f);
-  q.next.prev_n[j] = ToF4(p.prevN, p.medInter ? 1.f : 0.f);
+__device__ inline ExtPush ToExt(const uint4 &ids, uint32_t sid, uint32_t dim, float l0, const PathOut &p) {
+  ExtPush e;
+  e.o = ToF4(p.o, l0);
+  e.d = ToF4(p.d, p.eta);
+  e.beta = F4(p.beta);
+  e.ids = make_uint4(ids.x, ids.y, dim, (p.depth << 8) | p.flags);
+  e.aux = make_uint4(sid, p.pick, p.pass, p.med);
+  e.mis = p.mis;
+  e.pp = ToF4(p.prevP, 0.f);
+  e.pn = ToF4(p.prevN, p.medInter ? 1.f : 0.f);
+  return e;
 }
 
 // MISVolumetricPathIntegrator::LdMediumPoint (MISVolumetricPathIntegrator.cpp:23-69). `eh` is the
@@ -104,11 +106,15 @@ __global__ void __launch_bounds__(kBlock) k_shade_vol(DevScene sc, RenderParams 
                                                       AdjRefs ar) {
   __shared__ uint32_t stk[kLdsStack][kBlock];
   __shared__ TreeImp treeLds[kTreeLds];
+  __shared__ uint32_t pushLds[kBlock / 64 + 1];
   if (np) n = *np;
+  if (blockIdx.x * kBlock >= n) return;  // whole block idle: skip the LDS tree load
   LoadTreeLds(sc, treeLds);
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   EmitAcc eacc{{kNone, kNone}, {0.f, 0.f}};
-  if (i < n) {  // the adjoint's emission flush below needs every lane of the wave
+  bool pushed = false;
+  ExtPush ext;
+  if (i < n) {  // the queue push and the adjoint's emission flush below need every thread of the block
   const TraceCtx tc{stk, spillBase + (size_t)i * sc.spill_words};
   const bool corrected = rp.corrected != 0;
   const bool volumes = corrected && sc.num_media > 0;  // Scene::hasVolumes: never set as written
@@ -370,7 +376,7 @@ __global__ void __launch_bounds__(kBlock) k_shade_vol(DevScene sc, RenderParams 
           out.prevP = ToV3(ps.prev_p[i]); out.prevN = ToV3(ps.prev_n[i]);
           out.beta = beta;
           out.depth = depth;
-          Push(q, ids, sid, rng.dim, l0, out);
+          pushed = true;
         }
         push = false;
       } else {  // surface vertex (VolumetricPathIntegrator.cpp:45-90)
@@ -464,14 +470,16 @@ __global__ void __launch_bounds__(kBlock) k_shade_vol(DevScene sc, RenderParams 
       out.flags |= kFlagEmitOnly;
       out.flags &= ~kFlagRR;
     }
-    if (!kill || deferred) Push(q, ids, sid, rng.dim, l0, out);
+    pushed = !kill || deferred;
   }
+  if (pushed) ext = ToExt(ids, sid, rng.dim, l0, out);
   if (!IsBlack(Lacc, 1)) {
     float4 L = ss.L[sid];
     L.x += Lacc.c[0]; L.y += Lacc.c[1]; L.z += Lacc.c[2]; L.w += Lacc.c[3];
     ss.L[sid] = L;
   }
   }  // i < n
+  BlockPushExt(q.next, &q.counters[0], pushed, ext, pushLds);
   if constexpr (kAdjoint) EmitFlush(ar, eacc);
 }
 
