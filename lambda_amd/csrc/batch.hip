@@ -207,8 +207,8 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
           BatchLaunchShadow(s, scenes[j], b.ss, b.shadow, n, cout + 1, b.spill);
           nodes += 3;
         } else {
-          LaunchShadeVol((n + kBlock - 1) / kBlock, s, scenes[j], b.rp, b.ps[cur], b.ss, n, q, b.spill, nullptr, cin);
-          nodes += 2;
+          nodes += 1 + LaunchShadeVol((n + kBlock - 1) / kBlock, s, scenes[j], b.scp, b.rp, b.ps[cur], b.ss, n, q, b.spill,
+                                      nullptr, cin);
         }
       }
       BatchLaunchTrunc(s, b.ctr + 2 * iters, P.trunc.as<unsigned long long>());

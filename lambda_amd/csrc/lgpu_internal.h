@@ -375,11 +375,11 @@ void BatchLaunchAccumulate(hipStream_t s, const RenderParams &rp, const SampleSt
                            double *film, uint32_t *counts);
 
 // Volumetric shade stage (volume.hip): VolumetricPathIntegrator / MISVolumetricPathIntegrator;
-// with `adj`, the adjoint replay (adjoint.h).
+// with `adj`, the adjoint replay (adjoint.h). scp: the device's copy of sc. Returns the kernels launched.
 struct AdjRefs;
-void LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const RenderParams &rp, PathState ps,
-                    SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj = nullptr,
-                    const uint32_t *np = nullptr);
+uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const DevScene *scp, const RenderParams &rp,
+                        PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj = nullptr,
+                        const uint32_t *np = nullptr);
 // Utility-pass shade stage (utility.hip): DepthPass, NormalPass, AOVPass.
 void LaunchShadeUtility(uint32_t blocks, hipStream_t stream, const DevScene &sc, const RenderParams &rp, PathState ps,
                         SampleState ss, uint32_t n);

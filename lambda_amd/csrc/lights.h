@@ -134,9 +134,12 @@ __device__ inline Spec LightColour(const LightRec &L, const VmCtx &vm) {
   return S4(UpliftV(L.rgb[0], L.rgb[1], L.rgb[2], vm));
 }
 
+enum ShadowKind : uint32_t { kShadowSurface, kShadowPoint, kShadowEscape };
 struct ShadowSpec {
   V3 o, d;
-  float tmax;
+  float tmax;     // occlusion test's limit
+  float mag;      // distance to the light (kShadowEscape: unused)
+  uint32_t kind;  // a point on an emitter, a point or spot light, the environment
 };
 
 // Light::Sample_Li for the light kinds (MeshLight.cpp:22-41,134-151; PointLight.cpp:18-30;
@@ -144,11 +147,13 @@ struct ShadowSpec {
 // the shadow stage, `sh` receives the occlusion ray of Light::MutualVisibility / RayEscapes.
 // kInline = true: the ray is resolved here through `vc` (volumetric paths), Li carries Tr.
 // treeIdx (kInline = false only): the tree-light index of L when L is a tree light; its
-// triangle record in sc.tri_geo is then fetched together with L.
+// triangle record in sc.tri_geo is then fetched together with L. atMedium (kInline = false only): the
+// vertex is a medium interaction of the corrected estimator.
 template <bool kInline, bool kPrograms = true>
 __device__ inline Spec SampleLi(const DevScene &sc, const LightRec &L, const Hit &h, Ev &ev, Rng &rng, const VmCtx &vm,
-                                bool corrected, float &pdf, ShadowSpec &sh, const VisCtx *vc, uint32_t treeIdx = kNone) {
-  const bool noOff = kInline && vc->volumes && vc->atMedium;  // medium vertex: no surface offset
+                                bool corrected, float &pdf, ShadowSpec &sh, const VisCtx *vc, uint32_t treeIdx = kNone,
+                                bool atMedium = false) {
+  const bool noOff = kInline ? vc->volumes && vc->atMedium : atMedium;  // medium vertex: no surface offset
   Spec Tr = S(1.f);
   const bool geo = !kInline && treeIdx != kNone;
   float4 g0 = make_float4(0.f, 0.f, 0.f, 0.f), g1 = g0, g2 = g0;
@@ -183,6 +188,7 @@ __device__ inline Spec SampleLi(const DevScene &sc, const LightRec &L, const Hit
       const float mag = Mag(diff);
       ev.wi = diff / mag;
       sh.o = pS; sh.d = ev.wi; sh.tmax = (float)((double)mag - .00001);
+      sh.mag = mag; sh.kind = kShadowSurface;
       if (kInline && !Visible(sc, *vc, pS, ev.wi, mag, false, &Tr, vm)) { pdf = 0.f; return S(0.f); }
       float area;
       V3 normal;
@@ -214,6 +220,7 @@ __device__ inline Spec SampleLi(const DevScene &sc, const LightRec &L, const Hit
       const float mag = Mag(diff);
       ev.wi = diff / mag;
       sh.o = p; sh.d = ev.wi; sh.tmax = (float)((double)mag - .00001);
+      sh.mag = mag; sh.kind = kShadowPoint;
       if (kInline && !Visible(sc, *vc, p, ev.wi, mag, true, &Tr, vm)) { pdf = 0.f; return S(0.f); }
       pdf = 1.f;
       const float d2 = DistSq(pos, h.point);
@@ -247,6 +254,7 @@ __device__ inline Spec SampleLi(const DevScene &sc, const LightRec &L, const Hit
       sh.o = noOff ? h.point : h.point + h.normalG * kSurfaceEpsilon;
       sh.d = ev.wi;
       sh.tmax = INFINITY;
+      sh.mag = INFINITY; sh.kind = kShadowEscape;
       if (kInline && !Escapes(sc, *vc, sh.o, ev.wi, &Tr, vm)) { pdf = 0.f; return S(0.f); }
       ev.wiL = ToLocal(h, ev.wi);
       pdf /= 2 * kPi * kPi * sinT;
@@ -417,6 +425,40 @@ __device__ inline Spec VisibilityL(const DevScene &sc, const LightRec &L, V3 sp,
   }
   ls.pdf = 0.f;
   return S(0.f);
+}
+
+// VisibilityL of the corrected estimator with the ray left to the caller: sets ev.wi and sh, completes
+// ls.pdf and returns the factor beside the ray's transmittance. An environment is never reached this
+// way (its point sample's pdf is 0).
+__device__ inline Spec VisibilityDefer(const LightRec &L, V3 sp, Ev &ev, PartialLS &ls, ShadowSpec &sh) {
+  if (L.kind == kLightEnv) {
+    ls.pdf = 0.f;
+    return S(0.f);
+  }
+  const V3 diff = ls.point - sp;
+  const float mag = Mag(diff);
+  ev.wi = diff / mag;
+  sh.o = sp; sh.d = ev.wi; sh.tmax = (float)((double)mag - .00001);
+  sh.mag = mag;
+  if (L.kind == kLightMesh || L.kind == kLightTri) {
+    sh.kind = kShadowSurface;
+    const float dn = Dot(ls.normal, -ev.wi);
+    if (!(dn > 0)) {
+      ls.pdf = 0.f;
+      return S(0.f);
+    }
+    ls.pdf *= DistSq(sp, ls.point) / fabsf(dn);
+    return S(1.f);
+  }
+  sh.kind = kShadowPoint;
+  const float d2 = DistSq(ToV3(L.pos), sp);
+  if (L.kind != kLightSpot) return S(1.f) / d2;
+  const float cosT = Dot(-ev.wi, ToV3(L.axis));
+  float fall;
+  if (cosT < L.cos_cone) fall = 0.f;
+  else if (cosT > L.cos_falloff) fall = 1.f;
+  else { const float dd = (cosT - L.cos_cone) / (L.cos_falloff - L.cos_cone); fall = (dd * dd) * (dd * dd); }
+  return S(fall) / d2;
 }
 
 }  // namespace lgpu

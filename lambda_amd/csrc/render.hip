@@ -1146,7 +1146,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         else if (rp.integrator >= LGPU_INTEGRATOR_DEPTH)
           LaunchShadeUtility(Blocks(count), stream, dsc, rp, W.ps[cur], W.ss, count);
         else
-          LaunchShadeVol(Blocks(count), stream, dsc, rp, W.ps[cur], W.ss, count, q, W.spill_p, ap);
+          LaunchShadeVol(Blocks(count), stream, dsc, dscp, rp, W.ps[cur], W.ss, count, q, W.spill_p, ap);
         LGPU_HIP(hipGetLastError());
         LGPU_HIP(hipEventRecord(ev[4], stream));
         uint32_t cnt[2];

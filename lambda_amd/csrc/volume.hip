@@ -12,493 +12,238 @@
 //      equiangular triple with both medium points' direct light (MIS_VOLPATH);
 //   4. otherwise the surface vertex (NEE + BSDF sample) or a pass-through boundary;
 //   5. Russian roulette, then the continuation is appended to the next queue.
-// NEE visibility and the medium points' phase-sampled light lookups are traced inline.
-#include "adjoint.h"
-#include "host.h"
-#include "lights.h"
-#include "media.h"
-#include "queue.h"
-#include "shading.h"
-#include "trace.h"
+// Traced inline, all rays of a vertex run under the divergent masks of the shading code (8.5 of 64
+// lanes active in the fog room, measured), at the shading code's occupancy of two waves per SIMD.
+// For the corrected estimator the rays therefore run in kernels of their own: step 1 in k_vol_light
+// before, NEE visibility in k_vol_shadow after k_shade_vol, each with the block's rays gathered into
+// full waves. The faithful estimator and the adjoint replay need a ray's result inside the vertex and
+// trace inline. VALU instructions per wave and bounce in the fog room: 18,900 in one kernel; 2,000 here,
+// 2,100 in k_vol_light and 3,300 in k_vol_shadow. Fog room (301 x 211, 16 spp) 13.8 -> 10.1 ms, media
+// workload (1024 x 1024, 4 spp, 128^3 grid) 21.7 -> 17.3 ms.
+#include "volume_kernel.h"
 
 namespace lgpu {
 
 namespace {
 
-struct PathOut {  // continuation written to the next queue
-  V3 o, d;
-  float eta;
-  Spec beta;
-  uint32_t flags, depth, pick, pass, med;
-  float4 mis;
-  V3 prevP, prevN;
-  bool medInter = false;  // the vertex is a medium interaction (its deferred light lookup reads 3-D textures)
+// Scene::IntersectTr (Scene.cpp:45-81) as media.h's, with the hit records of the crossed surfaces
+// reduced to what the walk needs. t, u, v, bi: the last hit, o: the start of its segment.
+struct TrWalk {
+  V3 o;
+  float t, u, v, tFar = INFINITY;  // tFar: distance walked when the walk ended on a surface
+  uint32_t bi = kNone;
+  Spec Tr;
+  bool si = false, left = false;
 };
-
-__device__ inline ExtPush ToExt(const uint4 &ids, uint32_t sid, uint32_t dim, float l0, const PathOut &p) {
-  ExtPush e;
-  e.o = ToF4(p.o, l0);
-  e.d = ToF4(p.d, p.eta);
-  e.beta = F4(p.beta);
-  e.ids = make_uint4(ids.x, ids.y, dim, (p.depth << 8) | p.flags);
-  e.aux = make_uint4(sid, p.pick, p.pass, p.med);
-  e.mis = p.mis;
-  e.pp = ToF4(p.prevP, 0.f);
-  e.pn = ToF4(p.prevN, p.medInter ? 1.f : 0.f);
-  return e;
-}
-
-// MISVolumetricPathIntegrator::LdMediumPoint (MISVolumetricPathIntegrator.cpp:23-69). `eh` is the
-// event's hit: the path's hit in faithful mode (overwritten here as written), a copy in corrected.
-template <bool kPrograms>
-__device__ inline Spec LdMediumPoint(const DevScene &sc, const MediumRec &M, uint32_t med, Ev &ev, Hit &eh, V3 p,
-                                     PartialLS &ls, V3 refP, V3 refN, V3 *wiOut, Rng &rng, const VmCtx &vm,
-                                     bool corrected, const VisCtx &vc) {
-  const float partialLightPDF = corrected ? ls.selPdf : ls.pdf;
-  VmCtx vmm = vm;  // the phase-sampled light is looked up at a medium interaction
-  vmm.medium = 1;
-  eh.point = p;
-  Spec Li = S(0.f);
-  bool delta = false;
-  if (ls.light != kNone) {
-    const LightRec &LL = LightOf(sc, ls.light);
-    delta = LL.kind == kLightPoint || LL.kind == kLightSpot;
-    Li = ls.Le * VisibilityL(sc, LL, p, ev, eh, ls, vm, corrected, vc);
-  } else {
-    ls.pdf = 0.f;
-  }
-  const float lightPDF = ls.pdf;
-  Spec Ld = S(0.f);
-  if (lightPDF > 0 && !IsBlack(Li, vm.mode)) {
-    const float ph = PhaseHG(Dot(ev.wo, ev.wi), M.g);
-    if (ph > 0) {
-      const float w = (corrected && delta) ? 1.f : PowerHeuristic(lightPDF, ph);
-      Ld = Ld + Li * ph * w / lightPDF;
+__device__ inline void WalkTr(const DevScene &sc, TrWalk &w, V3 d, uint32_t med, float maxT, const VmCtx &vm,
+                              const TraceCtx &tc, bool haveFirst) {
+  float tFar = 0.f;
+  for (int k = 0; k < 256; ++k) {
+    uint32_t prim;
+    if (!(k == 0 && haveFirst) &&
+        !Trace4Closest(sc, w.o, d, 0.f, INFINITY, &w.t, &w.u, &w.v, &prim, &w.bi, tc.stk, tc.spill)) {
+      w.left = true;
+      return;
     }
+    const float4 *tp = reinterpret_cast<const float4 *>(sc.tris + w.bi);
+    const float4 w1 = tp[1], w2 = tp[2];
+    const V3 n = Norm(Cross(v3(w1.x, w1.y, w1.z), v3(w2.x, w2.y, w2.z)));
+    float seg = w.t;
+    tFar += seg;
+    const bool terminate = maxT >= 0.f && tFar > maxT;
+    if (terminate) {
+      const float delta = tFar - maxT;
+      tFar -= delta;
+      seg -= delta;
+    }
+    if (med != kNone) w.Tr = w.Tr * MediumTr(sc, sc.media[med], w.o, d, seg, vm);
+    const MaterialRec mat = sc.materials[sc.meshes[__float_as_uint(w1.w)].material];
+    w.tFar = seg;
+    if (terminate || mat.lobe != kNone || mat.emission != kNone) {
+      w.tFar = tFar;
+      w.si = true;
+      return;
+    }
+    med = GetMedium(mat, d, n);
+    const V3 p = v3(w.o.x + d.x * w.t, w.o.y + d.y * w.t, w.o.z + d.z * w.t);
+    w.o = p + n * (Dot(n, d) < 0 ? -kSurfaceEpsilon : kSurfaceEpsilon);
   }
-  const float u0 = rng.Get1D(), u1 = rng.Get1D();
-  V3 wi;
-  const float scatPdf = HGSample(M.g, ev.wo, &wi, u0, u1, corrected);
-  ev.wi = wi;
-  *wiOut = wi;
-  // corrected (the caller's hit record is a copy): without emissive meshes and an environment the
-  // phase-sampled ray reaches no light, its term adds zero, and its transmittance walk is skipped
-  if (corrected && !(sc.has_mesh_lights || sc.has_env)) return Ld;
-  Spec Tr = S(1.f);
-  uint32_t tbi = kNone;
-  const bool si = IntersectTr(sc, p, wi, med, -1.f, &Tr, vm, corrected, vc.tc, eh, tbi, nullptr, false);
-  if (scatPdf > 0) {
-    const Spec C = MisLight<kPrograms>(sc, ls.light, partialLightPDF, refP, refN, si, eh, tbi, wi, scatPdf, false, corrected, vmm,
-                            corrected);
-    Ld = Ld + (corrected ? C * Tr : C * Tr / scatPdf);  // the phase value is missing as written
-  }
-  return Ld;
 }
 
-// kPrograms: the scene has program sockets (DevScene::has_programs); without them the kernel is
-// compiled without the shader VM.
-// kAdjoint: the replay of the adjoint render (corrected estimator, RGB, VOLPATH): the same path
-// decisions and radiance as the primal launch, plus the gradient pieces of adjoint.h.
-// np: when set, the item count is read from this device counter (the grid covers an upper bound).
-template <bool kPrograms, bool kAdjoint>
-__global__ void __launch_bounds__(kBlock) k_shade_vol(DevScene sc, RenderParams rp, PathState ps, SampleState ss,
-                                                      uint32_t n, const uint32_t *np, Queues q, uint32_t *spillBase,
-                                                      AdjRefs ar) {
-  __shared__ uint32_t stk[kLdsStack][kBlock];
-  __shared__ TreeImp treeLds[kTreeLds];
-  __shared__ uint32_t pushLds[kBlock / 64 + 1];
-  if (np) n = *np;
-  if (blockIdx.x * kBlock >= n) return;  // whole block idle: skip the LDS tree load
-  LoadTreeLds(sc, treeLds);
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  EmitAcc eacc{{kNone, kNone}, {0.f, 0.f}};
-  bool pushed = false;
-  ExtPush ext;
-  if (i < n) {  // the queue push and the adjoint's emission flush below need every thread of the block
-  const TraceCtx tc{stk, spillBase + (size_t)i * sc.spill_words};
-  const bool corrected = rp.corrected != 0;
-  const bool volumes = corrected && sc.num_media > 0;  // Scene::hasVolumes: never set as written
-  const bool misVol = rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
-  const int mode = (int)rp.mode;
-  const uint4 ids = ps.ids[i];
-  const uint4 aux = ps.aux[i];
-  const uint32_t sid = aux.x;
-  const uint32_t flags = ids.w & 0xFFu;
-  const uint32_t depth = ids.w >> 8;
-  const uint32_t sideFlag = flags & kFlagSideNeg;
-  const float4 ro4 = ps.ray_o[i], rd4 = ps.ray_d[i];
-  const V3 ro = ToV3(ro4), rd = ToV3(rd4);
-  const float4 hr = ps.hit[i];
-  uint32_t bi = __float_as_uint(hr.w);
-  const bool hit = bi != kNone;
-  const uint32_t med = aux.w;
-  Spec beta = S4(ps.beta[i]);
-  Spec Lacc = S(0.f);
-  Spec adjd = S(0.f), rest = S(0.f);  // adjoint: loss gradient of the sample, radiance still to come
-  VisQuery vq{};
-  if constexpr (kAdjoint) {
-    adjd = AdjDelta(ar, ss.pixel[sid]);
-    rest = S4(ar.ltot[sid]) - S4(ss.L[sid]);
-  }
-  Rng rng;
-  rng.init(ids.x, ids.y, ids.z, rp.seed);
-  VmCtx vm;
-  vm.mode = mode;
+__device__ inline void WaveLengths(VmCtx &vm, const DevScene &sc, uint32_t mode, float l0) {
+  vm.mode = (int)mode;
   vm.texels = sc.texels; vm.textures = sc.textures; vm.consts = sc.consts; vm.code = sc.code;
-  const float l0 = ro4.w;
-  if (mode) {
-    for (int k = 0; k < 4; ++k) {
-      float l = l0 + 117.5f * (float)k;
-      if (l >= 830.f) l -= 470.f;
-      vm.lam[k] = l;
-    }
-  } else {
-    vm.lam[0] = vm.lam[1] = vm.lam[2] = vm.lam[3] = 0.f;
+  for (int k = 0; k < 4; ++k) {
+    float l = l0 + 117.5f * (float)k;
+    if (l >= 830.f) l -= 470.f;
+    vm.lam[k] = mode ? l : 0.f;
   }
   vm.woLy = 0.f;
-  vm.eta = rd4.w;
+  vm.eta = 0.f;
   vm.medium = 0;
+}
+
+// The block's threads whose flag is set, in order: their indices go to list, the count is returned.
+// Every thread of the block calls it; it begins and ends with a barrier. cnt: kBlock / 64 words.
+__device__ inline uint32_t BlockGather(bool take, uint32_t *cnt, uint16_t *list, uint32_t first) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const uint64_t m = __ballot(take);
+  __syncthreads();
+  if (lane == 0) cnt[wv] = (uint32_t)__popcll(m);
+  __syncthreads();
+  uint32_t before = first, total = first;
+  for (int w = 0; w < kBlock / 64; ++w) {
+    if (w < wv) before += cnt[w];
+    total += cnt[w];
+  }
+  if (take) list[before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)threadIdx.x;
+  __syncthreads();
+  return total;
+}
+
+// Step 1 for the block's paths that reach a light or cross a boundary: the light reached by the
+// previous vertex's sampled direction, added to the sample's radiance. Paths whose lookup has to walk
+// on through pass-through surfaces come first, so the walking waves are full.
+template <bool kPrograms>
+__global__ void __launch_bounds__(kBlock, 4)
+    k_vol_light(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
+                const uint32_t *np, uint32_t *spillBase) {
+  const DevScene &sc = *scp;
+  __shared__ uint32_t stk[kLdsStack][kBlock];
+  __shared__ uint32_t cnt[kBlock / 64];
+  __shared__ uint16_t list[kBlock];
+  if (np) n = *np;
+  const uint32_t base = blockIdx.x * kBlock, own = base + threadIdx.x;
+  if (base >= n) return;
+  bool walk = false, look = false;
+  if (own < n) {
+    const uint32_t flags = ps.ids[own].w, hb = __float_as_uint(ps.hit[own].w);
+    if (!(flags & (kFlagCamera | kFlagNoEmit))) {
+      if (hb == kNone) {
+        look = sc.has_env;
+      } else {
+        walk = (flags & kFlagTrMIS) && (sc.tris[hb].key & (kShadeKeys - 1)) == 1u;
+        look = !walk && sc.meshes[__float_as_uint(reinterpret_cast<const float4 *>(sc.tris + hb)[1].w)].mesh_light != kNone;
+      }
+    }
+  }
+  const uint32_t walks = BlockGather(walk, cnt, list, 0u);
+  const uint32_t total = BlockGather(look, cnt, list, walks);
+  if (threadIdx.x >= total) return;
+  const uint32_t i = base + list[threadIdx.x];
+  const uint4 aux = ps.aux[i];
+  const uint32_t flags = ps.ids[i].w;
+  const float4 ro4 = ps.ray_o[i], rd4 = ps.ray_d[i], hr = ps.hit[i];
+  const V3 rd = ToV3(rd4);
+  VmCtx vm;
+  WaveLengths(vm, sc, rp.mode, ro4.w);
+  vm.eta = rd4.w;
+  VmAtHit(vm, 0.f, 0.f, v3(0.f, 0.f, 0.f), v3(0.f, 0.f, 0.f));
+  TrWalk w;
+  w.o = ToV3(ro4);
+  w.t = hr.x; w.u = hr.y; w.v = hr.z; w.bi = __float_as_uint(hr.w);
+  w.Tr = S(1.f);
+  w.si = w.bi != kNone;
+  w.tFar = hr.x;
+  if ((flags & kFlagTrMIS) && w.si) {
+    w.si = false;
+    WalkTr(sc, w, rd, aux.w, -1.f, vm, TraceCtx{stk, spillBase + (size_t)own * sc.spill_words}, true);
+  }
   Hit h;
-  if (hit) ProcessHit(sc, ro, rd, hr.x, hr.y, hr.z, bi, corrected, h);
-  if (hit) VmAtHit(vm, h.u, h.v, h.point, h.normalS);
-  else VmAtHit(vm, 0.f, 0.f, v3(0.f, 0.f, 0.f), v3(0.f, 0.f, 0.f));
-  bool alive = true;
-
-  // ---- 1. light reached by the previous vertex's sampled direction. Without emissive meshes and
-  // an environment no light can be reached (MisLight finds none), so the term and its transmittance
-  // walk are skipped: they add zero.
-  if (!(flags & kFlagCamera) && !(flags & kFlagNoEmit) && !(sc.has_mesh_lights || sc.has_env)) {
-    if ((flags & kFlagEmitOnly) || !hit) alive = false;
-  } else if (!(flags & kFlagCamera) && !(flags & kFlagNoEmit)) {
-    const float4 mis = ps.mis[i];
-    bool si = hit;
-    Hit th = h;
-    uint32_t tbi = bi;
-    Spec Tr = S(1.f);
-    if ((flags & kFlagTrMIS) && hit) si = IntersectTr(sc, ro, rd, med, -1.f, &Tr, vm, corrected, tc, th, tbi, nullptr, true);
-    const float4 pn = ps.prev_n[i];
-    VmCtx vmm = vm;
-    vmm.medium = pn.w != 0.f;  // looked up for a medium interaction
-    const Spec C = MisLight<kPrograms>(sc, aux.y, mis.y, ToV3(ps.prev_p[i]), ToV3(pn), si, th, tbi, rd, mis.x,
-                            (flags & kFlagSpecular) != 0, false, vmm, corrected);
-    const Spec C1 = beta * (C * Tr * mis.w);
-    Lacc = Lacc + C1;
-    if constexpr (kAdjoint) {  // the light's intensity; the transmittance of the lookup's walk
-      const Spec X = adjd * C1;
-      if (si && sc.meshes[th.mesh].mesh_light != kNone) EmitAdd(sc, eacc, 0, sc.meshes[th.mesh].material, X);
-      if ((flags & kFlagTrMIS) && hit) TrGradWalk(sc, ar, ro, rd, med, -1.f, X, vm, tc);
-    }
-    if ((flags & kFlagEmitOnly) || !hit) alive = false;
-  } else if (!(flags & kFlagCamera) && !hit) {
-    alive = false;
+  if (w.si) {
+    ProcessHit(sc, w.o, rd, w.t, w.u, w.v, w.bi, true, h);
+    h.tFar = w.tFar;
   }
-  if (alive && (flags & kFlagRR)) beta = beta / S(1.f - ps.mis[i].z);  // VolumetricPathIntegrator.cpp:153
+  const float4 mis = ps.mis[i], pn = ps.prev_n[i];
+  vm.medium = pn.w != 0.f;  // looked up for a medium interaction
+  const Spec C = MisLight<kPrograms>(sc, aux.y, mis.y, ToV3(ps.prev_p[i]), ToV3(pn), w.si, h, w.bi, rd, mis.x,
+                                     (flags & kFlagSpecular) != 0, false, vm, true);
+  const Spec c = S4(ps.beta[i]) * (C * w.Tr * mis.w);
+  if (IsBlack(c, 1)) return;
+  float4 L = ss.L[aux.x];
+  L.x += c.c[0]; L.y += c.c[1]; L.z += c.c[2]; L.w += c.c[3];
+  ss.L[aux.x] = L;
+}
 
-  // ---- 2. bounce-0 emission (VolumetricPathIntegrator.cpp:32-39, 156-159)
-  if (alive && (flags & kFlagCamera)) {
-    if (!hit) {
-      if (sc.has_env) Lacc = Lacc + EnvLe(sc, rd, vm) * beta;
-      alive = false;
+// The visibility rays of the block's vertices (VolRays), slot by slot: a slot's rays are gathered
+// into full waves, and a path's second ray adds to its radiance after its first.
+__global__ void __launch_bounds__(kBlock, 4)
+    k_vol_shadow(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
+                 const uint32_t *np, uint32_t *spillBase, int slots) {
+  const DevScene &sc = *scp;
+  __shared__ uint32_t stk[kLdsStack][kBlock];
+  __shared__ uint32_t cnt[kBlock / 64];
+  __shared__ uint16_t list[kBlock];
+  if (np) n = *np;
+  const uint32_t base = blockIdx.x * kBlock, own = base + threadIdx.x;
+  if (base >= n) return;
+  const uint32_t ownBits = own < n ? __float_as_uint(ps.hit[own].z) : 0u;
+  const TraceCtx tc{stk, spillBase + (size_t)own * sc.spill_words};
+  for (int s = 0; s < slots; ++s) {
+    const uint32_t total = BlockGather((ownBits >> s) & 1u, cnt, list, 0u);
+    if (threadIdx.x >= total) continue;
+    const uint32_t i = base + list[threadIdx.x], sid = ps.aux[i].x;
+    const float4 o4 = (s ? ps.mis : ps.ray_o)[i], d4 = (s ? ps.prev_p : ps.ray_d)[i], hr = ps.hit[i];
+    const V3 d = ToV3(d4);
+    TrWalk w;
+    w.o = ToV3(o4);
+    w.Tr = S(1.f);
+    bool visible;
+    if (sc.num_media > 0) {
+      VmCtx vm;
+      WaveLengths(vm, sc, rp.mode, ss.lambda0[sid]);
+      WalkTr(sc, w, d, __float_as_uint(s ? hr.y : hr.x), o4.w, vm, tc, false);
+      const bool escape = ((__float_as_uint(hr.z) >> s) & kRayEscape) != 0u;
+      visible = escape ? !w.si : (w.left || w.tFar > d4.w);
     } else {
-      const MeshRec m = sc.meshes[h.mesh];
-      if (m.mesh_light != kNone && (!corrected || Dot(rd, h.normalG) < 0)) {
-        Spec Le = EmissionOf<kPrograms>(sc, h.mesh, vm) * sc.lights[m.mesh_light].intensity * kInvPi;
-        if (med != kNone) Le = Le * MediumTr(sc, sc.media[med], ro, rd, h.tFar, vm);
-        Lacc = Lacc + (corrected ? beta * Le : Le);  // beta taken as 1 as written
-        if constexpr (kAdjoint) {
-          const Spec X = adjd * (beta * Le);
-          EmitAdd(sc, eacc, 0, m.material, X);
-          if (med != kNone) TrGradSegment(sc, ar, sc.media[med], ro, rd, h.tFar, X, vm);
-        }
-      }
+      float t, u, v;
+      uint32_t prim, bi;
+      visible = !Trace<true, false>(sc, w.o, d, 0.f, o4.w, &t, &u, &v, &prim, &bi, tc.stk, tc.spill, nullptr);
     }
-  }
-
-  PathOut out;
-  bool push = false;
-  bool rrCheck = false;  // a scattering vertex happened: Russian roulette applies
-  if (alive) {
-    bool medInter = false;
-    // ---- 3. medium
-    if (med != kNone) {
-      const MediumRec M = sc.media[med];
-      Ev ev;
-      ev.wo = -rd;
-      ev.wi = rd;
-      ev.eta = rd4.w;
-      ev.woL = ev.wo;
-      ev.wiL = ev.wi;
-      ev.sidedness = sideFlag ? -1 : 1;
-      const VisCtx vc{tc, volumes, true, med, nullptr, v3(0, 0, 0), kAdjoint ? &vq : nullptr};
-      if (!misVol) {
-        const float u0 = rng.Get1D(), u1 = rng.Get1D();
-        const MediumSample ds = SampleDistance(sc, M, ro, rd, h.tFar, u0, u1, vm);
-        // every contribution from here on carries the distance sample's weight
-        if constexpr (kAdjoint) DistanceGrad(sc, ar, M, ro, rd, h.tFar, u0, u1, ds.inter, adjd * (rest - Lacc), vm);
-        beta = beta * ds.w;
-        if (ds.inter) {  // VolumetricPathIntegrator.cpp:99-148
-          medInter = true;
-          const V3 sp = ro + rd * ds.t;
-          h.point = sp;
-          vm.medium = 1;
-          vm.px = sp.x; vm.py = sp.y; vm.pz = sp.z;
-          const V3 refP = sp, refN = corrected ? v3(0, 0, 0) : h.normalS;
-          float lightDistPdf = 1.f;
-          const uint32_t pick = SampleLight(sc, refP, refN, rng, &lightDistPdf, treeLds, corrected);
-          Spec Li = S(0.f);
-          float lightPDF = 0.f;
-          bool delta = false;
-          if (pick != kNone) {
-            const LightRec &LL = LightOf(sc, pick);
-            delta = LL.kind == kLightPoint || LL.kind == kLightSpot;
-            ShadowSpec sh;
-            Li = SampleLi<true, kPrograms>(sc, LL, h, ev, rng, vm, corrected, lightPDF, sh, &vc);
-          }
-          lightPDF *= lightDistPdf;
-          Spec Ld = S(0.f);
-          if (lightPDF > 0 && !IsBlack(Li, mode)) {
-            const float ph = PhaseHG(Dot(ev.wo, ev.wi), M.g);
-            if (ph > 0) {
-              const float w = (corrected && delta) ? 1.f : PowerHeuristic(lightPDF, ph);
-              Ld = Ld + Li * ph * w / lightPDF;
-            }
-          }
-          if constexpr (kAdjoint) {  // the NEE contribution's light intensity and transmittance
-            const Spec X = adjd * (beta * Ld);
-            EmitAdd(sc, eacc, 1, EmitMaterial(sc, pick), X);
-            if (vq.valid) TrGradWalk(sc, ar, vq.o, vq.d, vq.med, vq.maxT, X, vm, tc);
-          }
-          const float hu0 = rng.Get1D(), hu1 = rng.Get1D();
-          V3 wi;
-          const float scatPdf = HGSample(M.g, ev.wo, &wi, hu0, hu1, corrected);
-          if (!(scatPdf > 0)) {
-            if (corrected) Lacc = Lacc + beta * Ld;
-          } else {
-            Lacc = Lacc + beta * Ld;
-            out.o = sp; out.d = wi; out.eta = rd4.w;
-            out.flags = kFlagTrMIS | sideFlag;
-            out.pick = pick;
-            out.mis = make_float4(scatPdf, lightDistPdf, 0.f, corrected ? 1.f : 1.f / scatPdf);
-            out.prevP = refP; out.prevN = refN;
-            out.medInter = true;
-            out.med = med;
-            push = true;
-            rrCheck = true;
-          }
-        }
-      } else {  // MISVolumetricPathIntegrator.cpp:92-147
-        const V3 refP = corrected ? ro : h.point, refN = corrected ? v3(0, 0, 0) : h.normalS;
-        PartialLS ls;
-        ls.pdf = 1.f;
-        ls.light = SampleLight(sc, refP, refN, rng, &ls.pdf, treeLds, corrected);
-        ls.selPdf = ls.pdf;
-        ls.point = v3(0, 0, 0);
-        ls.normal = v3(0, 0, 0);
-        if (ls.light != kNone) ls.Le = SamplePointL<kPrograms>(sc, LightOf(sc, ls.light), h, rng, vm, corrected, ls);
-        else { ls.pdf = 0.f; ls.Le = S(0.f); }
-        const int choice = rng.Get1D() > .5f ? 0 : 1;  // 0 distance, 1 equiangular
-        const float du0 = rng.Get1D(), du1 = rng.Get1D();
-        const float eps = rng.Get1D();
-        rng.Get1D();  // channel draw, unused (HomogeneousMedium.cpp:70)
-        rng.Get1D();
-        MediumSample sD, sE;  // one grid walk for both samples
-        SampleDistanceEquiangular(sc, M, ro, rd, h.tFar, du0, du1, h.point, ls.point, eps, vm, corrected, sD, sE);
-        const V3 mp0 = ro + rd * sD.t, mp1 = ro + rd * sE.t;
-        if (!corrected) {
-          if (!(sD.inter && sE.inter)) {
-            beta = beta * sD.w;
-          } else {
-            medInter = true;
-            const float pdfD2 = PdfDistanceAt(M, sE.D, sE.rho, vm, false);
-            const float pdfE2 = PdfEquiangular(ro, rd, ls.point, h.tFar, sD.t, false);
-            const float wD = PowerHeuristic(sD.pdf, pdfE2), wE = PowerHeuristic(sE.pdf, pdfD2);
-            V3 wi0, wi1;
-            Spec Ld = S(0.f);
-            Ld = Ld + LdMediumPoint<kPrograms>(sc, M, med, ev, h, mp0, ls, refP, refN, &wi0, rng, vm, false, vc) * sD.w * wD;
-            Ld = Ld + LdMediumPoint<kPrograms>(sc, M, med, ev, h, mp1, ls, refP, refN, &wi1, rng, vm, false, vc) * sE.w * wE;
-            Lacc = Lacc + Ld;  // beta missing as written
-            beta = beta * (choice == 0 ? sD.w : sE.w);
-            out.o = choice == 0 ? mp0 : mp1;
-            out.d = choice == 0 ? wi0 : wi1;
-            push = true;
-          }
-        } else {
-          // both points estimate direct light (power-heuristic MIS over the two distance
-          // techniques); the path continues with the distance sample
-          Spec Ld = S(0.f);
-          V3 wi0 = v3(0, 0, 0), wi1;
-          if (sD.inter) {
-            PartialLS l0 = ls;
-            Hit eh = h;
-            const float wD = PowerHeuristic(sD.pdf, PdfEquiangular(ro, rd, ls.point, h.tFar, sD.t, true));
-            Ld = Ld + LdMediumPoint<kPrograms>(sc, M, med, ev, eh, mp0, l0, refP, refN, &wi0, rng, vm, true, vc) * sD.w * wD;
-          }
-          if (sE.inter) {
-            PartialLS l1 = ls;
-            Hit eh = h;
-            const float wE = PowerHeuristic(sE.pdf, PdfDistanceAt(M, sE.D, sE.rho, vm, true));
-            Ld = Ld + LdMediumPoint<kPrograms>(sc, M, med, ev, eh, mp1, l1, refP, refN, &wi1, rng, vm, true, vc) * sE.w * wE;
-          }
-          Lacc = Lacc + beta * Ld;
-          beta = beta * sD.w;
-          if (sD.inter) {
-            medInter = true;
-            out.o = mp0;
-            out.d = wi0;
-            push = true;
-          }
-        }
-        if (push) {
-          out.eta = rd4.w;
-          out.flags = kFlagNoEmit | sideFlag;  // the phase-sampled light was looked up above
-          out.pick = kNone;
-          out.mis = make_float4(0.f, 0.f, 0.f, 0.f);
-          out.prevP = v3(0, 0, 0); out.prevN = v3(0, 0, 0);
-          out.med = med;
-          rrCheck = true;
-        }
-      }
-    }
-
-    // ---- 4. surface
-    if (!medInter) {
-      const MaterialRec mat = sc.materials[sc.meshes[h.mesh].material];
-      if (mat.lobe == kNone) {  // pass-through boundary (VolumetricPathIntegrator.cpp:91-97)
-        const uint32_t pass = aux.z + 1;
-        if (pass <= 1024) {
-          out.o = h.point + h.normalG * (Dot(h.normalG, rd) < 0 ? -kSurfaceEpsilon : kSurfaceEpsilon);
-          out.d = rd; out.eta = rd4.w;
-          out.flags = ((flags & kFlagCamera) ? kFlagCamera : kFlagNoEmit) | sideFlag;
-          out.pick = aux.y;
-          out.pass = pass;
-          out.med = GetMedium(mat, rd, h.normalG);
-          out.mis = ps.mis[i];
-          out.prevP = ToV3(ps.prev_p[i]); out.prevN = ToV3(ps.prev_n[i]);
-          out.beta = beta;
-          out.depth = depth;
-          pushed = true;
-        }
-        push = false;
-      } else {  // surface vertex (VolumetricPathIntegrator.cpp:45-90)
-        ShaderT<kPrograms> shd;
-        shd.sc = &sc;
-        shd.corrected = corrected;
-        Ev ev;
-        ev.wo = -rd;
-        ev.wi = rd;
-        ev.eta = rd4.w;
-        ev.woL = ToLocal(h, ev.wo);
-        ev.wiL = ToLocal(h, ev.wi);
-        ev.sidedness = (ev.woL.y > 0) ? 1 : -1;
-        vm.woLy = ev.woL.y;
-        shd.vm = vm;
-        const V3 shadeP = h.point, shadeN = h.normalS;
-        const VisCtx vc{tc, volumes, false, med, &mat, h.normalG, kAdjoint ? &vq : nullptr};
-        VertexGrad vg;
-        if constexpr (kAdjoint) VertexGradInit(shd, mat.lobe, vg);
-        float lightDistPdf = 1.f;
-        const uint32_t pick = SampleLight(sc, h.point, h.normalS, rng, &lightDistPdf, treeLds, corrected);
-        float lightPDF = 0.f;
-        Spec Li = S(0.f);
-        bool delta = false;
-        if (pick != kNone) {
-          const LightRec &LL = LightOf(sc, pick);
-          delta = LL.kind == kLightPoint || LL.kind == kLightSpot;
-          ShadowSpec sh;
-          Li = SampleLi<true, kPrograms>(sc, LL, h, ev, rng, vm, corrected, lightPDF, sh, &vc);
-        }
-        lightPDF *= lightDistPdf;
-        Spec cNee = S(0.f);
-        if (lightPDF > 0 && !IsBlack(Li, mode)) {
-          const Spec f0 = shd.F(mat.lobe, ev);
-          const Spec f = f0 * fabsf(ev.wiL.y);
-          const float sp = shd.Pdf(mat.lobe, ev.woL, ev.wiL);
-          if (!IsBlack(f, mode) && sp > 0) {
-            const float w = (corrected && delta) ? 1.f : PowerHeuristic(lightPDF, sp);
-            cNee = Li * f * w / lightPDF;
-            if constexpr (kAdjoint) {  // NEE: the BSDF at the light direction, intensity, transmittance
-              const Spec X = adjd * (beta * cNee);
-              VertexGradAdd(shd, ev, X, f0, vg);
-              EmitAdd(sc, eacc, 1, EmitMaterial(sc, pick), X);
-              if (vq.valid) TrGradWalk(sc, ar, vq.o, vq.d, vq.med, vq.maxT, X, vm, tc);
-            }
-          }
-        }
-        float scatPdf = 0.f;
-        bool spec = false;
-        const Spec fS = shd.Sample(mat.lobe, ev, h, rng, scatPdf, spec);
-        const Spec f = fS * fabsf(ev.wiL.y);
-        const uint32_t side = ev.sidedness < 0 ? kFlagSideNeg : 0u;
-        if (!(scatPdf > 0 && !IsBlack(f, mode))) {
-          if (corrected) Lacc = Lacc + beta * cNee;  // NEE is dropped by `break` as written
-          if constexpr (kAdjoint) VertexGradFlush(sc, ar, vm, vg);
-        } else {
-          Lacc = Lacc + beta * cNee;
-          if constexpr (kAdjoint) {  // continuation: everything later launches gather
-            if (!spec) VertexGradAdd(shd, ev, adjd * (rest - Lacc), fS, vg);
-            VertexGradFlush(sc, ar, vm, vg);
-          }
-          beta = beta * (f / scatPdf);
-          out.o = h.point; out.d = ev.wi; out.eta = ev.eta;
-          out.flags = (spec ? kFlagSpecular : 0u) | (volumes ? kFlagTrMIS : 0u) | side;
-          out.pick = pick;
-          out.mis = make_float4(scatPdf, lightDistPdf, 0.f, 1.f);
-          out.prevP = shadeP; out.prevN = shadeN;
-          out.med = GetMedium(mat, ev.wi, h.normalG);
-          push = true;
-          rrCheck = true;
-        }
-      }
-    }
-  }
-
-  // ---- 5. Russian roulette (VolumetricPathIntegrator.cpp:150-154) and the continuation
-  if (push) {
-    out.beta = beta;
-    out.depth = depth + 1;
-    out.pass = aux.z;
-    const bool deferred = !(out.flags & kFlagNoEmit);  // light lookup pending at the next hit
-    bool kill = false;
-    if (rrCheck && depth > rp.min_bounces) {
-      const float qrr = fmaxf(.05f, 1 - Luminance(beta, mode));
-      if (rng.Get1D() < qrr) kill = true;
-      else out.flags |= kFlagRR;
-      out.mis.z = qrr;
-    }
-    if (depth + 1 >= rp.max_bounces) kill = true;
-    if (kill) {
-      out.flags |= kFlagEmitOnly;
-      out.flags &= ~kFlagRR;
-    }
-    pushed = !kill || deferred;
-  }
-  if (pushed) ext = ToExt(ids, sid, rng.dim, l0, out);
-  if (!IsBlack(Lacc, 1)) {
+    if (!visible) continue;
+    const Spec c = S4((s ? ps.prev_n : ps.beta)[i]) * w.Tr;
     float4 L = ss.L[sid];
-    L.x += Lacc.c[0]; L.y += Lacc.c[1]; L.z += Lacc.c[2]; L.w += Lacc.c[3];
+    L.x += c.c[0]; L.y += c.c[1]; L.z += c.c[2]; L.w += c.c[3];
     ss.L[sid] = L;
   }
-  }  // i < n
-  BlockPushExt(q.next, &q.counters[0], pushed, ext, pushLds);
-  if constexpr (kAdjoint) EmitFlush(ar, eacc);
 }
 
 }  // namespace
 
-void LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const RenderParams &rp, PathState ps,
-                    SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj, const uint32_t *np) {
-  const AdjRefs ar = adj ? *adj : AdjRefs{};
-  const dim3 g(blocks), b(kBlock);
+void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
+                       PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np);
+void LaunchVolAdjoint(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
+                      PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs &ar,
+                      const uint32_t *np);
+
+uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const DevScene *scp, const RenderParams &rp,
+                        PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj,
+                        const uint32_t *np) {
+  const bool programs = sc.has_programs != 0;
   if (adj) {
-    if (sc.has_programs)
-      hipLaunchKernelGGL((k_shade_vol<true, true>), g, b, 0, stream, sc, rp, ps, ss, n, np, q, spill, ar);
-    else
-      hipLaunchKernelGGL((k_shade_vol<false, true>), g, b, 0, stream, sc, rp, ps, ss, n, np, q, spill, ar);
-  } else if (sc.has_programs) {
-    hipLaunchKernelGGL((k_shade_vol<true, false>), g, b, 0, stream, sc, rp, ps, ss, n, np, q, spill, ar);
-  } else {
-    hipLaunchKernelGGL((k_shade_vol<false, false>), g, b, 0, stream, sc, rp, ps, ss, n, np, q, spill, ar);
+    LaunchVolAdjoint(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, *adj, np);
+    return 1;
   }
+  if (!rp.corrected) {
+    LaunchVolFaithful(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, np);
+    return 1;
+  }
+  const dim3 g(blocks), b(kBlock);
+  const bool lights = sc.has_mesh_lights || sc.has_env;  // lights that a sampled direction can reach
+  const bool misVol = rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
+  const AdjRefs none{};
+  if (lights && programs) hipLaunchKernelGGL(k_vol_light<true>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill);
+  else if (lights) hipLaunchKernelGGL(k_vol_light<false>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill);
+  if (misVol && lights && programs)
+    hipLaunchKernelGGL((k_shade_vol<true, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+  else if (misVol && lights)
+    hipLaunchKernelGGL((k_shade_vol<false, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+  else if (programs)
+    hipLaunchKernelGGL((k_shade_vol<true, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+  else
+    hipLaunchKernelGGL((k_shade_vol<false, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+  hipLaunchKernelGGL(k_vol_shadow, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, misVol ? 2 : 1);
+  return lights ? 3 : 2;
 }
 
 }  // namespace lgpu

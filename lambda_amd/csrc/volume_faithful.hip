@@ -1,0 +1,14 @@
+// The volumetric shade kernel of the faithful estimator (volume.hip launches it).
+#include "volume_kernel.h"
+
+namespace lgpu {
+
+void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
+                 PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np) {
+  if (programs)
+    hipLaunchKernelGGL((k_shade_vol<true, kVolFaithful>), dim3(blocks), dim3(kBlock), 0, stream, scp, rp, ps, ss, n, np, q, spill, AdjRefs{});
+  else
+    hipLaunchKernelGGL((k_shade_vol<false, kVolFaithful>), dim3(blocks), dim3(kBlock), 0, stream, scp, rp, ps, ss, n, np, q, spill, AdjRefs{});
+}
+
+}  // namespace lgpu
