@@ -690,7 +690,11 @@ __global__ void __launch_bounds__(kBlock) k_accumulate_px(RenderParams rp, Sampl
                                                           double *film, uint32_t *counts) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= n || t >= npx) return;
-  double acc[3] = {0, 0, 0};
+  const uint32_t px = ss.pixel[t];
+  double *f = film + 3 * (size_t)px;
+  // the film's running sum goes on sample by sample, so the sums do not depend on how the samples were
+  // split into waves and passes
+  double acc[3] = {f[0], f[1], f[2]};
   uint32_t c = 0;
   for (uint32_t i = t; i < n; i += npx) {
     double rgb[3];
@@ -699,9 +703,7 @@ __global__ void __launch_bounds__(kBlock) k_accumulate_px(RenderParams rp, Sampl
     ++c;
     if (npx > n - i) break;  // next slot would pass n (also guards i + npx overflow)
   }
-  const uint32_t px = ss.pixel[t];
-  double *f = film + 3 * (size_t)px;
-  f[0] += acc[0]; f[1] += acc[1]; f[2] += acc[2];
+  f[0] = acc[0]; f[1] = acc[1]; f[2] = acc[2];
   counts[px] += c;
 }
 
