@@ -267,7 +267,7 @@ typedef struct lgpu_render_desc {
 
 typedef struct lgpu_render_stats {
   double ms_total;          /* host wall time of the call */
-  double ms_camera, ms_extend, ms_shade, ms_shadow; /* summed kernel times */
+  double ms_camera, ms_extend, ms_shade, ms_shadow; /* summed stage times (device clock at the stages' starts) */
   uint64_t samples;
   uint64_t extension_rays;
   uint64_t shadow_rays;

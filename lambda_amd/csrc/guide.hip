@@ -303,7 +303,9 @@ __device__ inline void QueryScalars(const GuideQuerySrc &src, const QueryRaw &r,
 template <bool kList>
 __global__ void __launch_bounds__(kInferBlock) k_guide_infer(const uint16_t *__restrict__ Wg, const float *__restrict__ Bg,
                                                                GuideQuerySrc src, uint32_t n, const uint32_t *np,
-                                                               uint32_t *__restrict__ bins, float2 *__restrict__ hdr) {
+                                                               uint32_t *__restrict__ bins, float2 *__restrict__ hdr,
+                                                               unsigned long long *stamp) {
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();  // the stage's start (BounceSlot)
   __shared__ __align__(16) uint16_t Wlds[kGuideWeights];
   __shared__ __align__(16) float Blds[kGuideBiases];
   constexpr int kPerBlock = (kInferBlock / 64) * 16 * kInferPT;
@@ -708,14 +710,14 @@ lgpu_status GuidePrepareWave(lgpu_guide g, const float bounds[6], uint64_t expec
 // `list` holds the bounce's guided vertices (`count` of them, at most `ub`), written by the
 // extension stage.
 lgpu_status GuideInfer(lgpu_guide g, const GuideRefs &refs, const PathState &ps, uint32_t ub, const uint32_t *list,
-                       const uint32_t *count, uint4 *bins, float2 *hdr, hipStream_t s) {
+                       const uint32_t *count, uint4 *bins, float2 *hdr, BounceSlot *slot, hipStream_t s) {
   GuideQuerySrc src{};
   src.ray_o = ps.ray_o; src.ray_d = ps.ray_d; src.hit = ps.hit; src.list = list; src.scalars = nullptr;
   for (int k = 0; k < 3; ++k) { src.bmin[k] = refs.bmin[k]; src.binv[k] = refs.binv[k]; }
   constexpr uint32_t kPerBlock = (kInferBlock / 64) * 16 * kInferPT;
   const uint32_t blocks = std::max<uint32_t>(1, std::min<uint32_t>((ub + kPerBlock - 1) / kPerBlock, g->infer_grid));
   hipLaunchKernelGGL(k_guide_infer<true>, dim3(blocks), dim3(kInferBlock), 0, s, g->wbf.as<uint16_t>(), g->bias.as<float>(), src, ub,
-                     count, reinterpret_cast<uint32_t *>(bins), hdr);
+                     count, reinterpret_cast<uint32_t *>(bins), hdr, slot ? &slot->infer : nullptr);
   LGPU_HIP(hipGetLastError());
   return LGPU_OK;
 }
@@ -871,7 +873,7 @@ extern "C" lgpu_status lgpu_guide_forward(lgpu_guide g, uint32_t n, const float 
   constexpr uint32_t kPerBlock = (kInferBlock / 64) * 16 * kInferPT;
   const uint32_t blocks = std::min<uint32_t>((n + kPerBlock - 1) / kPerBlock, g->infer_grid);
   hipLaunchKernelGGL(k_guide_infer<false>, dim3(blocks), dim3(kInferBlock), 0, s, g->wbf.as<uint16_t>(), g->bias.as<float>(), src, n,
-                     nullptr, dbins.as<uint32_t>(), dhdr.as<float2>());
+                     nullptr, dbins.as<uint32_t>(), dhdr.as<float2>(), nullptr);
   const hipError_t le = hipGetLastError();
   const hipError_t se = hipStreamSynchronize(s);
   LGPU_HIP(le);

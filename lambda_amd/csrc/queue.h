@@ -8,6 +8,21 @@
 
 namespace lgpu {
 
+// Device clock of a stage's start (BounceSlot), written by its first block; nothing without a slot.
+__device__ inline void Stamp(unsigned long long *t) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *t = wall_clock64();
+}
+// Copies a bounce's slot to pinned host memory; called by the first thread of the bounce's last kernel.
+// The host reads it after an event that follows the kernel.
+__device__ inline void Publish(const BounceSlot *slot, BounceSlot *host) {
+  host->next = slot->next;
+  host->shadow = slot->shadow;
+  host->extend = slot->extend;
+  host->infer = slot->infer;
+  host->shade = slot->shade;
+  host->shadows = slot->shadows;
+}
+
 struct ExtPush {
   float4 o, d, beta, mis, pp, pn;
   uint4 ids, aux;

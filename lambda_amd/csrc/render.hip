@@ -87,10 +87,18 @@ __device__ inline uint32_t TiledPixel(uint32_t j, uint32_t w, uint32_t h) {
   return ht * w + j;
 }
 
+// count, guideCount, host: a pipelined wave's first item count, its guide list's counter (null: none)
+// and the device clock at the wave's start.
 __global__ void __launch_bounds__(kBlock) k_camera(RenderParams rp, PathState ps, SampleState ss, uint32_t n,
-                                                   uint64_t base, const uint32_t *listPix, const uint32_t *listSmp) {
+                                                   uint64_t base, const uint32_t *listPix, const uint32_t *listSmp,
+                                                   uint32_t *count, uint32_t *guideCount, unsigned long long *host) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
+  if (count && i == 0) {
+    *count = n;
+    if (guideCount) *guideCount = 0u;
+    *host = wall_clock64();
+  }
   uint32_t pixel, sample;
   if (listPix) {
     pixel = listPix[i];
@@ -176,9 +184,14 @@ __device__ inline void GuideListAppend(bool take, uint32_t blockFirst, const Gui
 // device counter written by the previous stage (the grid then covers an upper bound of it).
 template <bool kCount, bool kList = false>
 __global__ void __launch_bounds__(kBlock) k_extend(DevScene sc, PathState ps, uint32_t n, const uint32_t *np,
-                                                   uint32_t *spill, unsigned long long *counts, GuideList gl) {
+                                                   uint32_t *spill, unsigned long long *counts, GuideList gl,
+                                                   BounceSlot *slot) {
   __shared__ uint32_t stk[kLdsStack][kBlock];
   __shared__ GuideListLds listLds;
+  if (slot && blockIdx.x == 0 && threadIdx.x == 0) {  // opens the bounce: its shading counts from zero
+    slot->next = slot->shadow = 0u;
+    slot->extend = wall_clock64();
+  }
   if (np) n = *np;
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   // with the list, every wave of a partial block arrives at it; whole idle blocks leave
@@ -216,8 +229,14 @@ __global__ void __launch_bounds__(kBlock) k_extend(DevScene sc, PathState ps, ui
 }
 
 __global__ void __launch_bounds__(kBlock) k_shadow(DevScene sc, SampleState ss, const ShadowRay *rays, uint32_t n,
-                                                   const uint32_t *np, uint32_t *spill) {
+                                                   const uint32_t *np, uint32_t *spill, BounceSlot *slot, BounceSlot *host,
+                                                   uint32_t *guideCount) {
   __shared__ uint32_t stk[kLdsStack][kBlock];
+  if (slot && blockIdx.x == 0 && threadIdx.x == 0) {  // closes the bounce
+    slot->shadows = wall_clock64();
+    Publish(slot, host);
+    if (guideCount) *guideCount = 0u;
+  }
   if (np) n = *np;
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
@@ -345,8 +364,9 @@ __device__ inline uint32_t Hash3(uint32_t a, uint32_t b, uint32_t c) {
 // strategies' pdfs for MIS with next-event estimation, and append training records.
 template <bool kCorrected, bool kPrograms, bool kGuided>
 __global__ void __launch_bounds__(kBlock, kPrograms ? 6 : 4) k_shade(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss,
-                                                  uint32_t n, const uint32_t *np, Queues q, GuideRefs gr) {
+                                                  uint32_t n, const uint32_t *np, Queues q, GuideRefs gr, BounceSlot *slot) {
   const DevScene &sc = *scp;
+  if (slot) Stamp(&slot->shade);
   __shared__ TreeImp treeLds[kTreeLds];
   __shared__ uint32_t keyStart[kShadeKeys];
   __shared__ uint16_t perm[kBlock];
@@ -660,8 +680,9 @@ __device__ inline void SampleRGB(const RenderParams &rp, float4 Lf, float l0, do
 // Per-sample film update for list-mode waves (any pixel may repeat): FP64 atomics, or the raw
 // per-sample record when `out` is set.
 __global__ void __launch_bounds__(kBlock) k_accumulate(RenderParams rp, SampleState ss, uint32_t n, double *film,
-                                                       uint32_t *counts, float *out) {
+                                                       uint32_t *counts, float *out, unsigned long long *host) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+  if (host && i == 0) *host = wall_clock64();
   if (i >= n) return;
   const float4 Lf = ss.L[i];
   const float l0 = ss.lambda0[i];
@@ -687,8 +708,9 @@ __global__ void __launch_bounds__(kBlock) k_accumulate(RenderParams rp, SampleSt
 // pixel's samples of the wave in sample order and updates its film entry once: each pixel has
 // one owner per launch (t < min(n, npx)), so no atomics are needed and the sum order is fixed.
 __global__ void __launch_bounds__(kBlock) k_accumulate_px(RenderParams rp, SampleState ss, uint32_t n, uint32_t npx,
-                                                          double *film, uint32_t *counts) {
+                                                          double *film, uint32_t *counts, unsigned long long *host) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
+  if (host && t == 0) *host = wall_clock64();
   if (t >= n || t >= npx) return;
   const uint32_t px = ss.pixel[t];
   double *f = film + 3 * (size_t)px;
@@ -737,15 +759,15 @@ __global__ void __launch_bounds__(kBlock) k_query(DevScene sc, const float4 *ray
 // ---------------------------------------------------------------- host side
 static void LaunchShade(bool corrected, bool programs, const GuideRefs *gr, uint32_t blocks, hipStream_t stream,
                         const DevScene *scp, const RenderParams &rp, const PathState &ps, const SampleState &ss, uint32_t n,
-                        const uint32_t *np, const Queues &q) {
+                        const uint32_t *np, const Queues &q, BounceSlot *slot = nullptr) {
   const dim3 g(blocks), b(kBlock);
   const GuideRefs none{};
-  if (gr && programs) hipLaunchKernelGGL((k_shade<true, true, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr);
-  else if (gr) hipLaunchKernelGGL((k_shade<true, false, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr);
-  else if (corrected && programs) hipLaunchKernelGGL((k_shade<true, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none);
-  else if (corrected) hipLaunchKernelGGL((k_shade<true, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none);
-  else if (programs) hipLaunchKernelGGL((k_shade<false, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none);
-  else hipLaunchKernelGGL((k_shade<false, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none);
+  if (gr && programs) hipLaunchKernelGGL((k_shade<true, true, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr, slot);
+  else if (gr) hipLaunchKernelGGL((k_shade<true, false, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr, slot);
+  else if (corrected && programs) hipLaunchKernelGGL((k_shade<true, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
+  else if (corrected) hipLaunchKernelGGL((k_shade<true, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
+  else if (programs) hipLaunchKernelGGL((k_shade<false, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
+  else hipLaunchKernelGGL((k_shade<false, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
 }
 
 // ---------------------------------------------------------------- batched renders (batch.hip)
@@ -766,12 +788,13 @@ void BatchLaunchTrunc(hipStream_t s, const uint32_t *cnt, unsigned long long *ac
 }
 void BatchLaunchCamera(hipStream_t s, const RenderParams &rp, const PathState &ps, const SampleState &ss, uint32_t n,
                        uint64_t base) {
-  hipLaunchKernelGGL(k_camera, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ps, ss, n, base, nullptr, nullptr);
+  hipLaunchKernelGGL(k_camera, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ps, ss, n, base, nullptr, nullptr,
+                     nullptr, nullptr, nullptr);
 }
 void BatchLaunchExtend(hipStream_t s, const DevScene &dsc, const PathState &ps, uint32_t ub, const uint32_t *np,
                        uint32_t *spill) {
   hipLaunchKernelGGL(k_extend<false>, dim3((ub + kBlock - 1) / kBlock), dim3(kBlock), 0, s, dsc, ps, ub, np, spill, nullptr,
-                     GuideList{});
+                     GuideList{}, nullptr);
 }
 void BatchLaunchShade(hipStream_t s, const DevScene *scp, const RenderParams &rp, const PathState &ps,
                       const SampleState &ss, uint32_t ub, const uint32_t *np, const Queues &q, bool programs) {
@@ -779,19 +802,21 @@ void BatchLaunchShade(hipStream_t s, const DevScene *scp, const RenderParams &rp
 }
 void BatchLaunchShadow(hipStream_t s, const DevScene &dsc, const SampleState &ss, const ShadowRay *rays, uint32_t ub,
                        const uint32_t *np, uint32_t *spill) {
-  hipLaunchKernelGGL(k_shadow, dim3((ub + kBlock - 1) / kBlock), dim3(kBlock), 0, s, dsc, ss, rays, ub, np, spill);
+  hipLaunchKernelGGL(k_shadow, dim3((ub + kBlock - 1) / kBlock), dim3(kBlock), 0, s, dsc, ss, rays, ub, np, spill, nullptr,
+                     nullptr, nullptr);
 }
 void BatchLaunchAccumulate(hipStream_t s, const RenderParams &rp, const SampleState &ss, uint32_t n, uint32_t npx,
                            double *film, uint32_t *counts) {
   const uint32_t m = n < npx ? n : npx;
-  hipLaunchKernelGGL(k_accumulate_px, dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ss, n, npx, film, counts);
+  hipLaunchKernelGGL(k_accumulate_px, dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ss, n, npx, film, counts,
+                     nullptr);
 }
 
 // Guiding hooks (guide.hip).
 lgpu_status GuidePrepareWave(lgpu_guide g, const float bounds[6], uint64_t expectedVertices, GuideRefs *refs,
                              const uint4 *bins, const float2 *hdr, hipStream_t s);
 lgpu_status GuideInfer(lgpu_guide g, const GuideRefs &refs, const PathState &ps, uint32_t ub, const uint32_t *list,
-                       const uint32_t *count, uint4 *bins, float2 *hdr, hipStream_t s);
+                       const uint32_t *count, uint4 *bins, float2 *hdr, BounceSlot *slot, hipStream_t s);
 lgpu_status GuideFinishWave(lgpu_guide g, const SampleState &ss, int mode, uint32_t trainSteps, uint64_t vertices,
                             hipStream_t s, uint32_t *records);
 uint64_t GuideExpectedVertices(lgpu_guide g);
@@ -812,15 +837,17 @@ struct Wave {
   uint32_t *counters_p = nullptr, *spill_p = nullptr;
   unsigned long long *tcount_p = nullptr;
   DevScene *scene_p = nullptr;
-  // pipelined path loop: device counter slots, their pinned host copies, per-slot stage events
+  // pipelined path loop: device slots, their pinned host copies, an event per slot (its bounce is
+  // done), and the device clock at a wave's start and at its film update (pinned)
   static constexpr int kSlots = 4;
-  uint32_t *hring = nullptr;
-  hipEvent_t pev[kSlots][6] = {};
+  BounceSlot *hring = nullptr;
+  unsigned long long *hwave = nullptr;
+  double ms_per_tick = 0.0;
+  hipEvent_t pev[kSlots] = {};
   ~Wave() {
     if (hring) (void)hipHostFree(hring);
-    for (auto &row : pev)
-      for (hipEvent_t &e : row)
-        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t &e : pev)
+      if (e) (void)hipEventDestroy(e);
   }
   // Device bytes one path in flight holds (both state buffers, sample state, shadow slot, spill;
   // guided: the bin table and header).
@@ -847,10 +874,15 @@ struct Wave {
       LGPU_HIP(gcount.alloc(256));
     }
     if (!hring) {
-      LGPU_HIP(hipHostMalloc((void **)&hring, 16 * kSlots, hipHostMallocDefault));
-      LGPU_HIP(ring.alloc(16 * kSlots));
-      for (auto &row : pev)
-        for (hipEvent_t &e : row) LGPU_HIP(hipEventCreate(&e));
+      int dev = 0, khz = 0;
+      LGPU_HIP(hipGetDevice(&dev));
+      LGPU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+      ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
+      LGPU_HIP(ring.alloc(sizeof(BounceSlot) * kSlots));
+      for (hipEvent_t &e : pev)
+        if (!e) LGPU_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      LGPU_HIP(hipHostMalloc((void **)&hring, sizeof(BounceSlot) * (kSlots + 1), hipHostMallocDefault));
+      hwave = reinterpret_cast<unsigned long long *>(hring + kSlots);
     }
     if (n <= cap) return LGPU_OK;
     cap = 0;  // until every part has grown: a failed growth leaves parts released
@@ -1010,6 +1042,13 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
   if (countTrav) LGPU_HIP(hipMemsetAsync(W.tcount_p, 0, 40, stream));
   lgpu_guide G = d->guide;
   GuideRefs gref{};
+  // pipelined loops: a bounce's last stage lasts until the next stamp
+  double *open = nullptr;
+  unsigned long long openAt = 0;
+  auto CloseStage = [&](unsigned long long at) {
+    if (open) *open += W.ms_per_tick * (double)(at - openAt);
+    open = nullptr;
+  };
   for (uint64_t base = 0; base < total; base += cap) {
     const uint32_t n = (uint32_t)std::min<uint64_t>(cap, total - base);
     int cur = 0;
@@ -1023,97 +1062,103 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
     for (int rep = 0; rep < (adj ? 2 : 1); ++rep) {  // adjoint: primal pass, then the replay
     const AdjRefs *ap = rep == 1 ? &adjW : nullptr;
     cur = 0;
-    LGPU_HIP(hipEventRecord(ev[0], stream));
-    hipLaunchKernelGGL(k_camera, dim3(Blocks(n)), dim3(kBlock), 0, stream, rp, W.ps[0], W.ss, n, base,
-                       listPix ? listPix + base : nullptr, listSmp ? listSmp + base : nullptr);
-    LGPU_HIP(hipGetLastError());
-    LGPU_HIP(hipEventRecord(ev[1], stream));
-    LGPU_HIP(hipStreamSynchronize(stream));
+    // path loops other than the direct and utility passes run ahead of the host (below)
+    const bool vol = rp.integrator == LGPU_INTEGRATOR_VOLPATH || rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
+    const bool pipelined = (rp.integrator == LGPU_INTEGRATOR_PATH || vol) && !bound;
+    BounceSlot *ring = pipelined ? W.ring.as<BounceSlot>() : nullptr;
     float ms;
-    LGPU_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
-    S.ms_camera += ms;
+    if (!pipelined) LGPU_HIP(hipEventRecord(ev[0], stream));
+    hipLaunchKernelGGL(k_camera, dim3(Blocks(n)), dim3(kBlock), 0, stream, rp, W.ps[0], W.ss, n, base,
+                       listPix ? listPix + base : nullptr, listSmp ? listSmp + base : nullptr,
+                       pipelined ? &ring[Wave::kSlots - 1].next : nullptr, G ? W.gcount.as<uint32_t>() : nullptr, W.hwave);
+    LGPU_HIP(hipGetLastError());
+    if (!pipelined) {
+      LGPU_HIP(hipEventRecord(ev[1], stream));
+      LGPU_HIP(hipStreamSynchronize(stream));
+      LGPU_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
+      S.ms_camera += ms;
+    }
     const uint32_t maxIter = 4 * (d->max_bounces + 2) + 1100;
-    if (rp.integrator == LGPU_INTEGRATOR_PATH && !bound) {
+    if (pipelined) {
       // Pipelined bounces: each stage reads its item count from the device counter the previous
       // stage wrote, the grids cover the last count the host has seen (counts never grow), and the
-      // host stays up to kLag bounces ahead, retiring them through pinned copies and events. No
-      // host round trip sits between two kernels.
+      // host stays up to kLag bounces ahead, retiring them through the published slots. No host
+      // round trip, copy, clear or timed event sits between two kernels.
       constexpr int kLag = 3;
       static_assert(kLag < Wave::kSlots, "a counter slot is reused only after its bounce retired");
-      uint32_t *ring = W.ring.as<uint32_t>();
-      LGPU_HIP(hipMemsetD32Async((hipDeviceptr_t)(ring + 4 * (Wave::kSlots - 1)), (int)n, 1, stream));  // bounce 0's input count
       uint32_t ub = n, live = n, issued = 0, retired = 0;
       bool done = false;
-      while (!(done && retired == issued)) {
-        if (!done && issued < maxIter && issued - retired < (uint32_t)kLag) {
+      while (!done) {
+        if (issued < maxIter && issued - retired < (uint32_t)kLag) {
           const int sl = (int)(issued % Wave::kSlots), prev = (int)((issued + Wave::kSlots - 1) % Wave::kSlots);
-          uint32_t *cin = ring + 4 * prev, *cout = ring + 4 * sl;
-          hipEvent_t *e = W.pev[sl];
-          LGPU_HIP(hipMemsetAsync(cout, 0, 8, stream));
+          uint32_t *cin = &ring[prev].next;
+          BounceSlot *slot = ring + sl, *host = W.hring + sl;
           // guided: the extension stage lists the bounce's guided vertices for the inference
           const GuideList gl{W.glist.as<uint32_t>(), W.gcount.as<uint32_t>(), G ? gref.max_depth : 0u};
-          if (G) LGPU_HIP(hipMemsetAsync(gl.count, 0, 4, stream));
-          LGPU_HIP(hipEventRecord(e[0], stream));
           if (countTrav && G)
             hipLaunchKernelGGL((k_extend<true, true>), dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ps[cur], ub, cin,
-                               W.spill_p, W.tcount_p, gl);
+                               W.spill_p, W.tcount_p, gl, slot);
           else if (countTrav)
             hipLaunchKernelGGL(k_extend<true>, dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ps[cur], ub, cin,
-                               W.spill_p, W.tcount_p, gl);
+                               W.spill_p, W.tcount_p, gl, slot);
           else if (G)
             hipLaunchKernelGGL((k_extend<false, true>), dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ps[cur], ub, cin,
-                               W.spill_p, W.tcount_p, gl);
+                               W.spill_p, W.tcount_p, gl, slot);
           else
             hipLaunchKernelGGL(k_extend<false>, dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ps[cur], ub, cin,
-                               W.spill_p, W.tcount_p, gl);
+                               W.spill_p, W.tcount_p, gl, slot);
           LGPU_HIP(hipGetLastError());
-          LGPU_HIP(hipEventRecord(e[1], stream));
           if (G) {  // the guide's distribution for the queue's guided vertices (before shading reads it)
             lgpu_status gs = GuideInfer(G, gref, W.ps[cur], ub, gl.list, gl.count, W.gbins.as<uint4>(),
-                                        W.ghdr.as<float2>(), stream);
+                                        W.ghdr.as<float2>(), slot, stream);
             if (gs != LGPU_OK) return gs;
           }
-          LGPU_HIP(hipEventRecord(e[5], stream));
-          Queues q{W.ps[cur ^ 1], W.shadow_p, cout};
-          LaunchShade(rp.corrected != 0, progs, G ? &gref : nullptr, Blocks(ub), stream, dscp, rp, W.ps[cur], W.ss, ub, cin, q);
+          Queues q{W.ps[cur ^ 1], W.shadow_p, &slot->next};
+          if (vol) {
+            LaunchShadeVol(Blocks(ub), stream, dsc, dscp, rp, W.ps[cur], W.ss, ub, q, W.spill_p, ap, cin, slot, host);
+          } else {
+            LaunchShade(rp.corrected != 0, progs, G ? &gref : nullptr, Blocks(ub), stream, dscp, rp, W.ps[cur], W.ss, ub, cin, q, slot);
+            LGPU_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_shadow, dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ss, W.shadow_p, ub,
+                               &slot->shadow, W.spill_p, slot, host, G ? W.gcount.as<uint32_t>() : nullptr);
+          }
           LGPU_HIP(hipGetLastError());
-          LGPU_HIP(hipEventRecord(e[2], stream));
-          hipLaunchKernelGGL(k_shadow, dim3(Blocks(ub)), dim3(kBlock), 0, stream, dsc, W.ss, W.shadow_p, ub,
-                             cout + 1, W.spill_p);
-          LGPU_HIP(hipGetLastError());
-          LGPU_HIP(hipEventRecord(e[3], stream));
-          LGPU_HIP(hipMemcpyAsync(W.hring + 4 * sl, cout, 8, hipMemcpyDeviceToHost, stream));
-          LGPU_HIP(hipEventRecord(e[4], stream));
+          LGPU_HIP(hipEventRecord(W.pev[sl], stream));
           cur ^= 1;
           ++issued;
           continue;
         }
         if (retired == issued) break;  // bounce limit reached without termination
         const int sl = (int)(retired % Wave::kSlots);
-        hipEvent_t *e = W.pev[sl];
-        LGPU_HIP(hipEventSynchronize(e[4]));
+        LGPU_HIP(hipEventSynchronize(W.pev[sl]));
+        const BounceSlot b = W.hring[sl];
+        if (retired == 0) S.ms_camera += W.ms_per_tick * (double)(b.extend - W.hwave[0]);
         ++retired;
-        if (done) continue;  // issued after the wave ended: processed no paths
-        const uint32_t c0 = W.hring[4 * sl], c1 = W.hring[4 * sl + 1];
-        float ms;
+        const uint32_t c0 = b.next, c1 = b.shadow;
         S.extension_rays += live;
         waveRays += live;
         S.launches_extend++;
         S.launches_shade++;
-        LGPU_HIP(hipEventElapsedTime(&ms, e[0], e[1]));
-        S.ms_extend += ms;
-        LGPU_HIP(hipEventElapsedTime(&ms, e[1], e[5]));
-        S.ms_guide_infer += ms;
-        LGPU_HIP(hipEventElapsedTime(&ms, e[5], e[2]));
-        S.ms_shade += ms;
-        if (c1) {
-          LGPU_HIP(hipEventElapsedTime(&ms, e[2], e[3]));
-          S.ms_shadow += ms;
-          S.shadow_rays += c1;
-          S.launches_shadow++;
+        CloseStage(retired == 1 ? W.hwave[1] : b.extend);  // a wave's last one ends where its film update began
+        S.ms_extend += W.ms_per_tick * (double)((G ? b.infer : b.shade) - b.extend);
+        if (G) S.ms_guide_infer += W.ms_per_tick * (double)(b.shade - b.infer);
+        if (vol && (ap || !rp.corrected)) {  // one kernel, its end stamped by the publishing one
+          S.ms_shade += W.ms_per_tick * (double)(b.shadows - b.shade);
+        } else if (vol) {  // one stage: the light lookups, shading and visibility rays
+          open = &S.ms_shade;
+          openAt = b.shade;
+        } else {
+          S.ms_shade += W.ms_per_tick * (double)(b.shadows - b.shade);
+          if (c1) {
+            open = &S.ms_shadow;
+            openAt = b.shadows;
+            S.shadow_rays += c1;
+            S.launches_shadow++;
+          }
         }
         if (c0 > live || c1 > live) return Fail(LGPU_ERR_STATE, "render: queue overflow");
         live = ub = c0;
+        // bounces issued past the last one process no paths; later work follows them on the stream
         if (c0 == 0) done = true;
       }
       if (!done) return Fail(LGPU_ERR_STATE, "render: path wave did not terminate");
@@ -1134,10 +1179,10 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         LGPU_HIP(hipEventRecord(ev[2], stream));
         if (countTrav)
           hipLaunchKernelGGL(k_extend<true>, dim3(Blocks(count)), dim3(kBlock), 0, stream, dsc, W.ps[cur], count, nullptr,
-                             W.spill_p, W.tcount_p, GuideList{});
+                             W.spill_p, W.tcount_p, GuideList{}, nullptr);
         else
           hipLaunchKernelGGL(k_extend<false>, dim3(Blocks(count)), dim3(kBlock), 0, stream, dsc, W.ps[cur], count, nullptr,
-                             W.spill_p, W.tcount_p, GuideList{});
+                             W.spill_p, W.tcount_p, GuideList{}, nullptr);
         LGPU_HIP(hipGetLastError());
         LGPU_HIP(hipEventRecord(ev[3], stream));
         Queues q{W.ps[cur ^ 1], W.shadow_p, W.counters_p};
@@ -1165,7 +1210,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         if (cnt[1]) {
           LGPU_HIP(hipEventRecord(ev[5], stream));
           hipLaunchKernelGGL(k_shadow, dim3(Blocks(cnt[1])), dim3(kBlock), 0, stream, dsc, W.ss, W.shadow_p,
-                             cnt[1], nullptr, W.spill_p);
+                             cnt[1], nullptr, W.spill_p, nullptr, nullptr, nullptr);
           LGPU_HIP(hipGetLastError());
           LGPU_HIP(hipEventRecord(ev[6], stream));
           LGPU_HIP(hipEventSynchronize(ev[6]));
@@ -1184,15 +1229,16 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
     const uint32_t npx = w * h;
     if (!listPix && !out && npx > 0)
       hipLaunchKernelGGL(k_accumulate_px, dim3(Blocks(std::min(n, npx))), dim3(kBlock), 0, stream, rp, W.ss, n, npx, film,
-                         counts);
+                         counts, W.hwave ? W.hwave + 1 : nullptr);
     else
       hipLaunchKernelGGL(k_accumulate, dim3(Blocks(n)), dim3(kBlock), 0, stream, rp, W.ss, n, film, counts,
-                         out ? out + 5 * base : nullptr);
+                         out ? out + 5 * base : nullptr, W.hwave ? W.hwave + 1 : nullptr);
     LGPU_HIP(hipGetLastError());
     }  // rep
     S.waves++;
   }
   LGPU_HIP(hipStreamSynchronize(stream));
+  if (W.hwave) CloseStage(W.hwave[1]);
   if (countTrav) {
     unsigned long long tc[5];
     LGPU_HIP(hipMemcpy(tc, W.tcount_p, 40, hipMemcpyDeviceToHost));

@@ -107,7 +107,8 @@ __device__ inline uint32_t BlockGather(bool take, uint32_t *cnt, uint16_t *list,
 template <bool kPrograms>
 __global__ void __launch_bounds__(kBlock, 4)
     k_vol_light(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
-                const uint32_t *np, uint32_t *spillBase) {
+                const uint32_t *np, uint32_t *spillBase, BounceSlot *slot) {
+  if (slot) Stamp(&slot->shade);
   const DevScene &sc = *scp;
   __shared__ uint32_t stk[kLdsStack][kBlock];
   __shared__ uint32_t cnt[kBlock / 64];
@@ -169,7 +170,8 @@ __global__ void __launch_bounds__(kBlock, 4)
 // into full waves, and a path's second ray adds to its radiance after its first.
 __global__ void __launch_bounds__(kBlock, 4)
     k_vol_shadow(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
-                 const uint32_t *np, uint32_t *spillBase, int slots) {
+                 const uint32_t *np, uint32_t *spillBase, int slots, BounceSlot *slot, BounceSlot *host) {
+  if (slot && blockIdx.x == 0 && threadIdx.x == 0) Publish(slot, host);  // closes the bounce
   const DevScene &sc = *scp;
   __shared__ uint32_t stk[kLdsStack][kBlock];
   __shared__ uint32_t cnt[kBlock / 64];
@@ -208,41 +210,47 @@ __global__ void __launch_bounds__(kBlock, 4)
   }
 }
 
+// Closes a bounce whose shading is a single kernel.
+__global__ void k_publish(BounceSlot *slot, BounceSlot *host) {
+  slot->shadows = wall_clock64();
+  Publish(slot, host);
+}
+
 }  // namespace
 
 void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
-                       PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np);
+                       PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np,
+                       BounceSlot *slot);
 void LaunchVolAdjoint(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
                       PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs &ar,
-                      const uint32_t *np);
+                      const uint32_t *np, BounceSlot *slot);
 
 uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const DevScene *scp, const RenderParams &rp,
                         PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj,
-                        const uint32_t *np) {
+                        const uint32_t *np, BounceSlot *slot, BounceSlot *host) {
   const bool programs = sc.has_programs != 0;
-  if (adj) {
-    LaunchVolAdjoint(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, *adj, np);
-    return 1;
-  }
-  if (!rp.corrected) {
-    LaunchVolFaithful(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, np);
+  if (adj || !rp.corrected) {
+    if (adj) LaunchVolAdjoint(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, *adj, np, slot);
+    else LaunchVolFaithful(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, np, slot);
+    if (slot) hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, stream, slot, host);
     return 1;
   }
   const dim3 g(blocks), b(kBlock);
   const bool lights = sc.has_mesh_lights || sc.has_env;  // lights that a sampled direction can reach
   const bool misVol = rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
   const AdjRefs none{};
-  if (lights && programs) hipLaunchKernelGGL(k_vol_light<true>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill);
-  else if (lights) hipLaunchKernelGGL(k_vol_light<false>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill);
+  BounceSlot *first = lights ? nullptr : slot;  // the stage's start is stamped by its first kernel
+  if (lights && programs) hipLaunchKernelGGL(k_vol_light<true>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, slot);
+  else if (lights) hipLaunchKernelGGL(k_vol_light<false>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, slot);
   if (misVol && lights && programs)
-    hipLaunchKernelGGL((k_shade_vol<true, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+    hipLaunchKernelGGL((k_shade_vol<true, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
   else if (misVol && lights)
-    hipLaunchKernelGGL((k_shade_vol<false, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+    hipLaunchKernelGGL((k_shade_vol<false, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
   else if (programs)
-    hipLaunchKernelGGL((k_shade_vol<true, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
+    hipLaunchKernelGGL((k_shade_vol<true, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
   else
-    hipLaunchKernelGGL((k_shade_vol<false, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none);
-  hipLaunchKernelGGL(k_vol_shadow, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, misVol ? 2 : 1);
+    hipLaunchKernelGGL((k_shade_vol<false, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
+  hipLaunchKernelGGL(k_vol_shadow, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, misVol ? 2 : 1, slot, host);
   return lights ? 3 : 2;
 }
 

@@ -164,7 +164,8 @@ __device__ inline Spec LdMediumPoint(const DevScene &sc, const MediumRec &M, uin
 template <bool kPrograms, VolMode kMode>
 __global__ void __launch_bounds__(kBlock, kMode == kVolSplit ? 4 : 2)
     k_shade_vol(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
-                const uint32_t *np, Queues q, uint32_t *spillBase, AdjRefs ar) {
+                const uint32_t *np, Queues q, uint32_t *spillBase, AdjRefs ar, BounceSlot *slot) {
+  if (slot) Stamp(&slot->shade);
   constexpr bool kAdjoint = kMode == kVolAdjoint;
   constexpr bool kSplit = kMode == kVolSplit || kMode == kVolSplitLookup;  // rays resolved by k_vol_light, k_vol_shadow
   constexpr bool kTraces = kMode != kVolSplit;
