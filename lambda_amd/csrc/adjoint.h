@@ -101,7 +101,7 @@ __device__ inline float DLambdaDAlpha(bool ggx, V3 w, float a) {
 
 // Derivatives of one leaf lobe's f at ev: gA[c] = d f_c / d albedo_c, gR[c] = d f_c / d roughness
 // (the roughness socket's value, before Microfacet.cpp:49-55's mapping when the lobe applies it).
-template <bool kPrograms>
+template <int kPrograms>
 __device__ inline void LeafDerivs(const ShaderT<kPrograms> &shd, const Lobe &L, const Ev &ev, Spec *gA, Spec *gR) {
   *gA = S(0.f);
   *gR = S(0.f);
@@ -150,7 +150,7 @@ struct VertexGrad {
   uint32_t leaf[2];  // lobe indices (kNone: unused)
   float mixw[2];
 };
-template <bool kPrograms>
+template <int kPrograms>
 __device__ inline void VertexGradInit(const ShaderT<kPrograms> &shd, uint32_t root, VertexGrad &vg) {
   for (int l = 0; l < 2; ++l)
     for (int k = 0; k < 4; ++k) { vg.alb[l][k] = 0.f; vg.rough[l][k] = 0.f; }
@@ -166,7 +166,7 @@ __device__ inline void VertexGradInit(const ShaderT<kPrograms> &shd, uint32_t ro
 }
 // Adds the gradient of contributions X (delta-weighted, carrying f = the lobe tree's value at ev)
 // through f.
-template <bool kPrograms>
+template <int kPrograms>
 __device__ inline void VertexGradAdd(const ShaderT<kPrograms> &shd, const Ev &ev, Spec X, Spec f, VertexGrad &vg) {
   Spec q;  // X / f per channel
   for (int c = 0; c < 4; ++c) q.c[c] = (c < 3 && f.c[c] != 0.f) ? X.c[c] / f.c[c] : 0.f;

@@ -142,7 +142,8 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
     ShadowRay *shadow;
     uint32_t *spill, *ctr;
     const DevScene *scp;
-    bool path, programs;
+    bool path;
+    int programs;
   };
   std::vector<Job> jobs(J);
   for (uint32_t j = 0; j < J; ++j) {
@@ -164,7 +165,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
     b.ctr = P.ctr.as<uint32_t>() + (size_t)ctrWords * j;
     b.scp = P.scenes.as<DevScene>() + j;
     b.path = d[j].integrator == LGPU_INTEGRATOR_PATH;
-    b.programs = scenes[j].has_programs != 0;
+    b.programs = (int)scenes[j].has_programs;
   }
   Branches &br = BranchesOf(dev);
   { lgpu_status s = br.init(); if (s != LGPU_OK) return s; }

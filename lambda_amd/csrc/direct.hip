@@ -14,7 +14,7 @@ namespace lgpu {
 
 namespace {
 
-template <bool kPrograms>
+template <int kPrograms>
 __device__ inline Spec EmissionAt(const DevScene &sc, const Hit &lh, VmCtx vm) {
   VmAtHit(vm, lh.u, lh.v, lh.point, lh.normalS);
   return EmissionOf<kPrograms>(sc, lh.mesh, vm) * sc.lights[sc.meshes[lh.mesh].mesh_light].intensity * kInvPi;
@@ -52,9 +52,9 @@ __device__ inline float PdfLiRay(const DevScene &sc, uint32_t pick, const Hit &h
   return 0.f;
 }
 
-// kPrograms: the scene has program sockets (DevScene::has_programs); without them the kernel is
+// kPrograms: what the scene's sockets need (DevScene::has_programs); without any the kernel is
 // compiled without the shader VM.
-template <bool kPrograms>
+template <int kPrograms>
 __global__ void __launch_bounds__(kBlock) k_shade_direct(DevScene sc, RenderParams rp, PathState ps, SampleState ss,
                                                          uint32_t n, Queues q, uint32_t *spillBase) {
   __shared__ uint32_t stk[kLdsStack][kBlock];
@@ -204,9 +204,9 @@ __global__ void __launch_bounds__(kBlock) k_shade_direct(DevScene sc, RenderPara
 void LaunchShadeDirect(uint32_t blocks, hipStream_t stream, const DevScene &sc, const RenderParams &rp, PathState ps,
                        SampleState ss, uint32_t n, Queues q, uint32_t *spill) {
   if (sc.has_programs)
-    hipLaunchKernelGGL(k_shade_direct<true>, dim3(blocks), dim3(kBlock), 0, stream, sc, rp, ps, ss, n, q, spill);
+    hipLaunchKernelGGL(k_shade_direct<kVmPrograms>, dim3(blocks), dim3(kBlock), 0, stream, sc, rp, ps, ss, n, q, spill);
   else
-    hipLaunchKernelGGL(k_shade_direct<false>, dim3(blocks), dim3(kBlock), 0, stream, sc, rp, ps, ss, n, q, spill);
+    hipLaunchKernelGGL(k_shade_direct<kNoPrograms>, dim3(blocks), dim3(kBlock), 0, stream, sc, rp, ps, ss, n, q, spill);
 }
 
 }  // namespace lgpu

@@ -186,8 +186,17 @@ enum SocketKind : uint32_t {
   kSockColour = 1,      // value.rgb; as spectrum: RGB in RGB mode, uplift at the hero wavelengths
   kSockBlackbody = 2,   // value.rgb = RGB-mode blackbody, value.w = temperature
   kSockVec2 = 3,        // value.xy (anisotropic roughness)
-  kSockProgram = 4      // run code[prog_off .. +prog_len); result in r[res]
+  kSockProgram = 4,     // run code[prog_off .. +prog_len); result in r[res]
+  kSockTexture = 5      // one bilinear lookup of texture prog_off, read as prog_len (TexRead) says; res: channel
 };
+enum TexRead : uint32_t {
+  kTexSpectrum = 0,     // the texel's colour as a spectrum
+  kTexChannel = 1,      // one channel, as a real (as spectrum: broadcast)
+  kTexReal = 2          // the texel's colour as a real
+};
+// What a scene's sockets need (DevScene::has_programs); the shading kernels specialise on it: nothing
+// beyond constants, texture lookups, or the shader VM.
+enum ProgramLevel : int { kNoPrograms = 0, kTexPrograms = 1, kVmPrograms = 2 };
 struct Socket {
   float value[4];
   uint32_t kind;
@@ -324,7 +333,7 @@ struct DevScene {
   const float *density;      // grid densities of all media
   uint32_t num_media;
   uint32_t spill_words;      // per-thread traversal-stack words beyond the LDS part this tree can need
-  uint32_t has_programs;     // some socket runs VM code (shading kernels specialise on it)
+  uint32_t has_programs;     // ProgramLevel of the scene's sockets (shading kernels specialise on it)
   unsigned long long *voxel_count;  // non-null in counting renders: voxels visited by grid walks
   const AdjLobe *adj_lobes;  // per lobe: texture bindings for the adjoint render
 };
@@ -383,7 +392,7 @@ void BatchLaunchCamera(hipStream_t s, const RenderParams &rp, const PathState &p
 void BatchLaunchExtend(hipStream_t s, const DevScene &dsc, const PathState &ps, uint32_t ub, const uint32_t *np,
                        uint32_t *spill);
 void BatchLaunchShade(hipStream_t s, const DevScene *scp, const RenderParams &rp, const PathState &ps,
-                      const SampleState &ss, uint32_t ub, const uint32_t *np, const Queues &q, bool programs);
+                      const SampleState &ss, uint32_t ub, const uint32_t *np, const Queues &q, int programs);
 void BatchLaunchShadow(hipStream_t s, const DevScene &dsc, const SampleState &ss, const ShadowRay *rays, uint32_t ub,
                        const uint32_t *np, uint32_t *spill);
 void BatchLaunchAccumulate(hipStream_t s, const RenderParams &rp, const SampleState &ss, uint32_t n, uint32_t npx,

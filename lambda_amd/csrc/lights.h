@@ -116,7 +116,7 @@ __device__ inline void TriAreaNormal(V3 v0, V3 v1, V3 v2, float *area, V3 *norma
   *area = Mag(c) * .5f;
   if (normal) *normal = c / (*area * 2.f);
 }
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 __device__ inline Spec EmissionOf(const DevScene &sc, uint32_t mesh, const VmCtx &vm) {
   const MaterialRec m = sc.materials[sc.meshes[mesh].material];
   if (m.emission == kNone) return S(0.f);
@@ -149,7 +149,7 @@ struct ShadowSpec {
 // treeIdx (kInline = false only): the tree-light index of L when L is a tree light; its
 // triangle record in sc.tri_geo is then fetched together with L. atMedium (kInline = false only): the
 // vertex is a medium interaction of the corrected estimator.
-template <bool kInline, bool kPrograms = true>
+template <bool kInline, int kPrograms = kVmPrograms>
 __device__ inline Spec SampleLi(const DevScene &sc, const LightRec &L, const Hit &h, Ev &ev, Rng &rng, const VmCtx &vm,
                                 bool corrected, float &pdf, ShadowSpec &sh, const VisCtx *vc, uint32_t treeIdx = kNone,
                                 bool atMedium = false) {
@@ -285,7 +285,7 @@ __device__ inline float PdfLiHit(const DevScene &sc, const LightRec &L, V3 wi, c
 // ray's hit (si: it hit something); refP/refN is the corrected light-selection reference point.
 // Returns Le * w; the caller applies f or Tr and 1/pdf. envNoLightPdf: the light technique
 // cannot produce the environment (point sampling at medium vertices, corrected).
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 __device__ inline Spec MisLight(const DevScene &sc, uint32_t l, float lightDistPdf, V3 refP, V3 refN, bool si, const Hit &h,
                                 uint32_t bi, V3 rd, float scatPdf, bool specular, bool envNoLightPdf, VmCtx vm,
                                 bool corrected) {
@@ -329,7 +329,7 @@ struct PartialLS {
 };
 // Light::SamplePoint (MeshLight.cpp:66-81,166-180; PointLight.cpp:40-44; Spotlight.cpp:50-54;
 // EnvironmentLight.cpp:69-74). Faithful writes the sampled uv into the event hit (h, vm) as written.
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 __device__ inline Spec SamplePointL(const DevScene &sc, const LightRec &L, Hit &h, Rng &rng, VmCtx &vm, bool corrected,
                                     PartialLS &ls) {
   switch (L.kind) {

@@ -310,8 +310,8 @@ __device__ inline void BlockPush(const Queues &q, bool pushE, const ExtPush &e, 
 
 // kCorrected: the estimator mode (rp.corrected) as a template argument, so each instantiation
 // carries only its own mode's branches.
-// kPrograms: the scene has program sockets (DevScene::has_programs); without them the kernel is
-// compiled without the shader VM, spills little, and runs best at four waves per SIMD (with the
+// kPrograms: what the scene's sockets need (DevScene::has_programs); without program sockets the kernel
+// is compiled without the shader VM, spills little, and runs best at four waves per SIMD (with the
 // VM's call frames and call-site spills, six).
 // Guide table of one path slot: GuideBin / sampling over the 128 bin weights (sum `tot`).
 __device__ inline float GuideBinPdf(const uint8_t *tab, float tot, uint32_t bin) {
@@ -362,8 +362,8 @@ __device__ inline uint32_t Hash3(uint32_t a, uint32_t b, uint32_t c) {
 // kGuided (corrected estimator only): guidable vertices sample one-sample MIS of the learned
 // guide (the path slot's bin table, inferred after extension) and the BSDF, evaluate both
 // strategies' pdfs for MIS with next-event estimation, and append training records.
-template <bool kCorrected, bool kPrograms, bool kGuided>
-__global__ void __launch_bounds__(kBlock, kPrograms ? 6 : 4) k_shade(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss,
+template <bool kCorrected, int kPrograms, bool kGuided>
+__global__ void __launch_bounds__(kBlock, kPrograms == kVmPrograms ? 6 : 4) k_shade(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss,
                                                   uint32_t n, const uint32_t *np, Queues q, GuideRefs gr, BounceSlot *slot) {
   const DevScene &sc = *scp;
   if (slot) Stamp(&slot->shade);
@@ -757,17 +757,22 @@ __global__ void __launch_bounds__(kBlock) k_query(DevScene sc, const float4 *ray
 }
 
 // ---------------------------------------------------------------- host side
-static void LaunchShade(bool corrected, bool programs, const GuideRefs *gr, uint32_t blocks, hipStream_t stream,
+template <bool kCorrected, bool kGuided>
+static void LaunchShadeAs(int programs, const dim3 &g, hipStream_t stream, const DevScene *scp, const RenderParams &rp,
+                          const PathState &ps, const SampleState &ss, uint32_t n, const uint32_t *np, const Queues &q,
+                          const GuideRefs &gr, BounceSlot *slot) {
+  const dim3 b(kBlock);
+  if (programs == kVmPrograms) hipLaunchKernelGGL((k_shade<kCorrected, kVmPrograms, kGuided>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, gr, slot);
+  else if (programs == kTexPrograms) hipLaunchKernelGGL((k_shade<kCorrected, kTexPrograms, kGuided>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, gr, slot);
+  else hipLaunchKernelGGL((k_shade<kCorrected, kNoPrograms, kGuided>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, gr, slot);
+}
+static void LaunchShade(bool corrected, int programs, const GuideRefs *gr, uint32_t blocks, hipStream_t stream,
                         const DevScene *scp, const RenderParams &rp, const PathState &ps, const SampleState &ss, uint32_t n,
                         const uint32_t *np, const Queues &q, BounceSlot *slot = nullptr) {
-  const dim3 g(blocks), b(kBlock);
-  const GuideRefs none{};
-  if (gr && programs) hipLaunchKernelGGL((k_shade<true, true, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr, slot);
-  else if (gr) hipLaunchKernelGGL((k_shade<true, false, true>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, *gr, slot);
-  else if (corrected && programs) hipLaunchKernelGGL((k_shade<true, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
-  else if (corrected) hipLaunchKernelGGL((k_shade<true, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
-  else if (programs) hipLaunchKernelGGL((k_shade<false, true, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
-  else hipLaunchKernelGGL((k_shade<false, false, false>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, none, slot);
+  const dim3 g(blocks);
+  if (gr) LaunchShadeAs<true, true>(programs, g, stream, scp, rp, ps, ss, n, np, q, *gr, slot);
+  else if (corrected) LaunchShadeAs<true, false>(programs, g, stream, scp, rp, ps, ss, n, np, q, GuideRefs{}, slot);
+  else LaunchShadeAs<false, false>(programs, g, stream, scp, rp, ps, ss, n, np, q, GuideRefs{}, slot);
 }
 
 // ---------------------------------------------------------------- batched renders (batch.hip)
@@ -797,7 +802,7 @@ void BatchLaunchExtend(hipStream_t s, const DevScene &dsc, const PathState &ps, 
                      GuideList{}, nullptr);
 }
 void BatchLaunchShade(hipStream_t s, const DevScene *scp, const RenderParams &rp, const PathState &ps,
-                      const SampleState &ss, uint32_t ub, const uint32_t *np, const Queues &q, bool programs) {
+                      const SampleState &ss, uint32_t ub, const uint32_t *np, const Queues &q, int programs) {
   LaunchShade(true, programs, nullptr, (ub + kBlock - 1) / kBlock, s, scp, rp, ps, ss, ub, np, q);
 }
 void BatchLaunchShadow(hipStream_t s, const DevScene &dsc, const SampleState &ss, const ShadowRay *rays, uint32_t ub,
@@ -1035,7 +1040,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
   // whose address reaches out-of-line functions is copied into every lane's scratch.
   LGPU_HIP(hipMemcpyAsync(W.scene_p, &dsc, sizeof(DevScene), hipMemcpyHostToDevice, stream));
   const DevScene *dscp = W.scene_p;
-  const bool progs = dsc.has_programs != 0;
+  const int progs = (int)dsc.has_programs;
   hipEvent_t *ev = dev->ev;
   lgpu_render_stats S;
   std::memset(&S, 0, sizeof(S));

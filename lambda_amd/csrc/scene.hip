@@ -1099,9 +1099,6 @@ lgpu_status CommitScene(lgpu_scene s, uint32_t strategy) {
   d.num_lights = (uint32_t)lights.size();
   d.num_media = (uint32_t)media.size();
   d.spill_words = spillWords;
-  d.has_programs = 0;
-  for (const Socket &k : sockets)
-    if (k.kind != kSockScalar && k.kind != kSockColour && k.kind != kSockBlackbody && k.kind != kSockVec2) d.has_programs = 1;
   d.has_env = hasEnv;
   d.has_mesh_lights = 0;  // as MisLight reads it: some mesh record names a light
   for (const MeshRec &m : meshes)
@@ -1242,6 +1239,31 @@ lgpu_status CommitScene(lgpu_scene s, uint32_t strategy) {
   // ------------------------------------------------ upload
   lgpu_status st;
 #define UP(vec, field) if ((st = Upload(s, vec, &d.field)) != LGPU_OK) return st
+  // Program sockets that are one texture lookup through at most one conversion become texture sockets
+  // (after everything above that reads their code).
+  d.has_programs = kNoPrograms;
+  for (Socket &k : sockets) {
+    if (k.kind != kSockProgram) continue;
+    uint32_t read = kNone;
+    if (k.prog_len == 1 || k.prog_len == 2) {
+      const Instr &a = code[k.prog_off], &b = code[k.prog_off + k.prog_len - 1];
+      const bool whole = k.prog_len == 1, conv = !whole && b.a == a.dst;
+      const bool ends = b.dst == k.res;
+      if (a.op == kOpTex && conv && ends && b.op == kOpToSpectrum && b.c == kColour) read = kTexSpectrum;
+      if (a.op == kOpTex && conv && ends && b.op == kOpToReal && b.c == kColour) read = kTexReal;
+      const bool lookup = a.op == kOpTex || a.op == kOpTexChannel;  // read as a scalar: one channel (kOpTex: the first)
+      if (lookup && conv && ends && b.op == kOpToSpectrum && b.c == kScalar) read = kTexChannel;
+      if (lookup && whole && ends && k.res_type == kScalar) read = kTexChannel;
+      if (read != kNone) {
+        k.kind = kSockTexture;
+        k.prog_off = a.imm;
+        k.prog_len = read;
+        k.res = read == kTexChannel && a.op == kOpTexChannel ? a.c : 0u;
+      }
+    }
+    d.has_programs = std::max<uint32_t>(d.has_programs, read == kNone ? kVmPrograms : kTexPrograms);
+  }
+
   UP(bb.nodes, nodes);
   UP(bb.nodes4, nodes4);
   UP(btris, tris);

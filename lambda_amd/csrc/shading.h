@@ -220,7 +220,7 @@ __device__ inline void RoughDielectricEval(V3 wo, V3 wi, float alpha, float ior,
 
 // ---------------------------------------------------------------- lobes
 // kPrograms: as for the socket readers (false only on scenes without program sockets).
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 struct ShaderT {
   const DevScene *sc;
   VmCtx vm;

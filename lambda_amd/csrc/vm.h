@@ -334,11 +334,27 @@ static __host__ __device__ __attribute__((noinline)) float4 RunProgram(const VmC
   return r[res];
 }
 
-// Socket readers. kPrograms = false compiles them without the VM: for shading kernels launched
-// only on scenes without program sockets (DevScene::has_programs == 0), where the out-of-line
-// RunProgram calls would otherwise shape the whole kernel's register allocation.
+// The lookup of a texture socket. Out of line (a shading kernel reads sockets at dozens of places),
+// with scalar arguments: a reference to the context would put it into per-lane scratch.
+static __host__ __device__ __attribute__((noinline)) float4 TexLookup(const float *texels, const uint4 *textures,
+                                                                       uint32_t tex, float u, float v) {
+  const uint4 t = textures[tex];
+  float px[4];
+  TexBilinear(texels + t.w, t.x, t.y, t.z, Fract(u), Fract(v), px);
+  return make_float4(px[0], px[1], px[2], px[3]);
+}
+LGPU_HD float4 SocketTexel(const Socket &s, const VmCtx &c) {
+  return TexLookup(c.texels, c.textures, s.prog_off, c.u, c.v);
+}
+
+// Socket readers. kPrograms below kVmPrograms compiles them without the VM, kNoPrograms without
+// texture lookups too: for shading kernels launched only on scenes that need no more
+// (DevScene::has_programs), where the out-of-line RunProgram calls would otherwise shape the whole
+// kernel's register allocation. A socket that is one texture lookup through at most one conversion (an
+// image texture wired straight to a lobe) is no program: interpreted, its values went through a
+// register file in scratch.
 // Socket read as a spectrum (GetAsSpectrum).
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 LGPU_HD Spec SocketSpectrum(const Socket &s, const VmCtx &c) {
   switch (s.kind) {
     case kSockScalar: return S(s.value[0]);
@@ -355,28 +371,43 @@ LGPU_HD Spec SocketSpectrum(const Socket &s, const VmCtx &c) {
       return o;
     }
     case kSockVec2: return S(0.f);
+    case kSockTexture:
+      if constexpr (kPrograms != kNoPrograms) {
+        const float4 t = SocketTexel(s, c);
+        return s.prog_len == kTexChannel ? S(Comp(t, s.res)) : S4(UpliftV(t.x, t.y, t.z, c));
+      }
+      return S(0.f);
     default:
-      if constexpr (kPrograms) return S4(RunProgram(c, s.prog_off, s.prog_len, s.res));
+      if constexpr (kPrograms == kVmPrograms) return S4(RunProgram(c, s.prog_off, s.prog_len, s.res));
       else return S(0.f);
   }
 }
 // Socket read as a real (GetAs<Real>).
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 LGPU_HD float SocketReal(const Socket &s, const VmCtx &c) {
   switch (s.kind) {
     case kSockScalar: return s.value[0];
     case kSockVec2: return (s.value[0] + s.value[1]) * .5f;
+    case kSockTexture:
+      if constexpr (kPrograms != kNoPrograms) {
+        const float4 t = SocketTexel(s, c);
+        return s.prog_len == kTexChannel ? Comp(t, s.res) : AsRealV(t, kColour, c.mode);
+      }
+      return 0.f;
     case kSockProgram:
-      if constexpr (kPrograms) return RunProgram(c, s.prog_off, s.prog_len, s.res).x;
+      if constexpr (kPrograms == kVmPrograms) return RunProgram(c, s.prog_off, s.prog_len, s.res).x;
       else return 0.f;
   }
   return s.value[0];
 }
 // Microfacet roughness: scalar (isotropic) or vec2 (anisotropic) (Microfacet.cpp:57-69).
-template <bool kPrograms = true>
+template <int kPrograms = kVmPrograms>
 LGPU_HD void SocketRoughness(const Socket &s, const VmCtx &c, float *a, float *b) {
   if (s.kind == kSockVec2) { *a = s.value[0]; *b = s.value[1]; return; }
-  if constexpr (kPrograms) {
+  if constexpr (kPrograms != kNoPrograms) {
+    if (s.kind == kSockTexture) { *a = *b = SocketReal<kPrograms>(s, c); return; }
+  }
+  if constexpr (kPrograms == kVmPrograms) {
     if (s.kind == kSockProgram) {
       const float4 v = RunProgram(c, s.prog_off, s.prog_len, s.res);
       if (s.res_type == kVec2) { *a = v.x; *b = v.y; }

@@ -104,7 +104,7 @@ __device__ inline uint32_t BlockGather(bool take, uint32_t *cnt, uint16_t *list,
 // Step 1 for the block's paths that reach a light or cross a boundary: the light reached by the
 // previous vertex's sampled direction, added to the sample's radiance. Paths whose lookup has to walk
 // on through pass-through surfaces come first, so the walking waves are full.
-template <bool kPrograms>
+template <int kPrograms>
 __global__ void __launch_bounds__(kBlock, 4)
     k_vol_light(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
                 const uint32_t *np, uint32_t *spillBase, BounceSlot *slot) {
@@ -218,17 +218,17 @@ __global__ void k_publish(BounceSlot *slot, BounceSlot *host) {
 
 }  // namespace
 
-void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
+void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, int programs, const RenderParams &rp,
                        PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np,
                        BounceSlot *slot);
-void LaunchVolAdjoint(uint32_t blocks, hipStream_t stream, const DevScene *scp, bool programs, const RenderParams &rp,
+void LaunchVolAdjoint(uint32_t blocks, hipStream_t stream, const DevScene *scp, int programs, const RenderParams &rp,
                       PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs &ar,
                       const uint32_t *np, BounceSlot *slot);
 
 uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc, const DevScene *scp, const RenderParams &rp,
                         PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const AdjRefs *adj,
                         const uint32_t *np, BounceSlot *slot, BounceSlot *host) {
-  const bool programs = sc.has_programs != 0;
+  const int programs = (int)sc.has_programs;
   if (adj || !rp.corrected) {
     if (adj) LaunchVolAdjoint(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, *adj, np, slot);
     else LaunchVolFaithful(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, np, slot);
@@ -240,16 +240,27 @@ uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc,
   const bool misVol = rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
   const AdjRefs none{};
   BounceSlot *first = lights ? nullptr : slot;  // the stage's start is stamped by its first kernel
-  if (lights && programs) hipLaunchKernelGGL(k_vol_light<true>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, slot);
-  else if (lights) hipLaunchKernelGGL(k_vol_light<false>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, slot);
-  if (misVol && lights && programs)
-    hipLaunchKernelGGL((k_shade_vol<true, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
-  else if (misVol && lights)
-    hipLaunchKernelGGL((k_shade_vol<false, kVolSplitLookup>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
-  else if (programs)
-    hipLaunchKernelGGL((k_shade_vol<true, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
-  else
-    hipLaunchKernelGGL((k_shade_vol<false, kVolSplit>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first);
+#define LGPU_VOL_LIGHT(kLevel) \
+  hipLaunchKernelGGL(k_vol_light<kLevel>, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, slot)
+#define LGPU_VOL_SHADE(kLevel, kMode) \
+  hipLaunchKernelGGL((k_shade_vol<kLevel, kMode>), g, b, 0, stream, scp, rp, ps, ss, n, np, q, spill, none, first)
+  if (lights) {
+    if (programs == kVmPrograms) LGPU_VOL_LIGHT(kVmPrograms);
+    else if (programs == kTexPrograms) LGPU_VOL_LIGHT(kTexPrograms);
+    else LGPU_VOL_LIGHT(kNoPrograms);
+  }
+  if (misVol && lights) {
+    if (programs) LGPU_VOL_SHADE(kVmPrograms, kVolSplitLookup);
+    else LGPU_VOL_SHADE(kNoPrograms, kVolSplitLookup);
+  } else if (programs == kVmPrograms) {
+    LGPU_VOL_SHADE(kVmPrograms, kVolSplit);
+  } else if (programs == kTexPrograms) {
+    LGPU_VOL_SHADE(kTexPrograms, kVolSplit);
+  } else {
+    LGPU_VOL_SHADE(kNoPrograms, kVolSplit);
+  }
+#undef LGPU_VOL_LIGHT
+#undef LGPU_VOL_SHADE
   hipLaunchKernelGGL(k_vol_shadow, g, b, 0, stream, scp, rp, ps, ss, n, np, spill, misVol ? 2 : 1, slot, host);
   return lights ? 3 : 2;
 }

@@ -104,7 +104,7 @@ __device__ inline ExtPush ToExt(const uint4 &ids, uint32_t sid, uint32_t dim, fl
 // event's hit: the path's hit in faithful mode (overwritten here as written), a copy in corrected.
 // Split: the visibility ray goes to `sh` and the light's term without the ray's transmittance to
 // `nee`; the result holds the phase-sampled lookup only.
-template <bool kPrograms, VolMode kMode>
+template <int kPrograms, VolMode kMode>
 __device__ inline Spec LdMediumPoint(const DevScene &sc, const MediumRec &M, uint32_t med, Ev &ev, Hit &eh, V3 p,
                                      PartialLS &ls, V3 refP, V3 refN, V3 *wiOut, Rng &rng, const VmCtx &vm,
                                      bool corrected, const VisCtx &vc, ShadowSpec *sh, Spec *nee) {
@@ -155,13 +155,13 @@ __device__ inline Spec LdMediumPoint(const DevScene &sc, const MediumRec &M, uin
   return Ld;
 }
 
-// kPrograms: the scene has program sockets (DevScene::has_programs); without them the kernel is
-// compiled without the shader VM. The scene record comes through a pointer: a by-value argument whose
+// kPrograms: what the scene's sockets need (DevScene::has_programs); without program sockets the kernel
+// is compiled without the shader VM. The scene record comes through a pointer: a by-value argument whose
 // address reaches out-of-line functions is copied into every lane's scratch.
 // kVolAdjoint: the replay of the adjoint render (RGB, VOLPATH): the same path decisions and radiance
 // as the primal launch, plus the gradient pieces of adjoint.h.
 // np: when set, the item count is read from this device counter (the grid covers an upper bound).
-template <bool kPrograms, VolMode kMode>
+template <int kPrograms, VolMode kMode>
 __global__ void __launch_bounds__(kBlock, kMode == kVolSplit ? 4 : 2)
     k_shade_vol(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
                 const uint32_t *np, Queues q, uint32_t *spillBase, AdjRefs ar, BounceSlot *slot) {
