@@ -64,6 +64,7 @@ lgpu_status lgpu_device_destroy(lgpu_device d) {
   (void)hipStreamSynchronize(d->stream);
   if (d->wave && d->wave_free) d->wave_free(d->wave);
   if (d->batch && d->batch_free) d->batch_free(d->batch);
+  if (d->copier && d->copier_free) d->copier_free(d->copier);
   // guides still alive lose their device memory here; their handles stay valid for destroy
   if (d->guide_orphan)
     for (void *g : d->guides) d->guide_orphan(g);
@@ -399,8 +400,8 @@ lgpu_status lgpu_film_read(lgpu_film f, double *rgb, uint32_t *counts) {
   std::lock_guard<std::mutex> lk(f->dev->mu);
   LGPU_HIP(hipSetDevice(f->dev->device));
   LGPU_HIP(hipStreamSynchronize(f->dev->stream));
-  if (rgb) LGPU_HIP(hipMemcpy(rgb, f->sum.ptr, 24ull * f->width * f->height, hipMemcpyDeviceToHost));
-  if (counts) LGPU_HIP(hipMemcpy(counts, f->count.ptr, 4ull * f->width * f->height, hipMemcpyDeviceToHost));
+  if (rgb) LGPU_HIP(CopyToHost(f->dev, rgb, f->sum.ptr, 24ull * f->width * f->height));
+  if (counts) LGPU_HIP(CopyToHost(f->dev, counts, f->count.ptr, 4ull * f->width * f->height));
   return LGPU_OK;
 }
 // The inverse of lgpu_film_read: the film's sums and counts from host arrays (a saved film to
@@ -411,9 +412,9 @@ lgpu_status lgpu_film_write(lgpu_film f, const double *rgb, const uint32_t *coun
   LGPU_HIP(hipSetDevice(f->dev->device));
   LGPU_HIP(hipStreamSynchronize(f->dev->stream));
   const size_t n = (size_t)f->width * f->height;
-  LGPU_HIP(hipMemcpy(f->sum.ptr, rgb, 24ull * n, hipMemcpyHostToDevice));
+  LGPU_HIP(CopyToDevice(f->dev, f->sum.ptr, rgb, 24ull * n));
   if (counts) {
-    LGPU_HIP(hipMemcpy(f->count.ptr, counts, 4ull * n, hipMemcpyHostToDevice));
+    LGPU_HIP(CopyToDevice(f->dev, f->count.ptr, counts, 4ull * n));
   } else {
     std::vector<uint32_t> ones(n, 1u);
     LGPU_HIP(hipMemcpy(f->count.ptr, ones.data(), 4ull * n, hipMemcpyHostToDevice));

@@ -109,7 +109,7 @@ lgpu_status lgpu_film_denoise(lgpu_film colour, lgpu_film albedo, lgpu_film norm
   LGPU_HIP(hipSetDevice(colour->dev->device));
   (void)hipGetLastError();
   const hipStream_t st = colour->dev->stream;
-  DevBuf ca, cb, ab, nb;
+  DevBuf &ca = colour->dev->work[0], &cb = colour->dev->work[1], &ab = colour->dev->work[2], &nb = colour->dev->work[3];
   LGPU_HIP(ca.alloc(16ull * n));
   LGPU_HIP(cb.alloc(16ull * n));
   const dim3 g1((n + 255) / 256), b1(256);
@@ -142,7 +142,8 @@ lgpu_status lgpu_film_denoise(lgpu_film colour, lgpu_film albedo, lgpu_film norm
   hipLaunchKernelGGL(k_dn_to_film, g1, b1, 0, st, src, demod ? ab.as<float4>() : nullptr, demod ? 1u : 0u, n,
                      out->sum.as<double>(), out->count.as<uint32_t>());
   const hipError_t le = hipGetLastError();
-  const hipError_t se = hipStreamSynchronize(st);  // before the buffers leave scope
+  const hipError_t se = hipStreamSynchronize(st);  // before the buffers are used by another call
+  colour->dev->trim_work();
   LGPU_HIP(le);
   LGPU_HIP(se);
   return LGPU_OK;

@@ -72,7 +72,12 @@ struct HostLight {
 };
 
 // Film::ToRGBTexture into host memory (4 floats per pixel); the caller holds the device mutex.
-lgpu_status FilmToRgba(lgpu_film f, float *rgba);
+// pinned: rgba is page-locked (copied to directly).
+lgpu_status FilmToRgba(lgpu_film f, float *rgba, bool pinned = false);
+// Copies between a caller's array and device memory, after the work already on the device's stream; the
+// data has arrived on return (host_copy.hip). The caller holds the device mutex.
+hipError_t CopyToHost(lgpu_device d, void *host, const void *dev, size_t n);
+hipError_t CopyToDevice(lgpu_device d, void *dev, const void *host, size_t n);
 
 }  // namespace lgpu
 
@@ -85,9 +90,17 @@ struct lgpu_device_s {
   void (*wave_free)(void *) = nullptr;
   void *batch = nullptr;              // capture streams and events of batched renders
   void (*batch_free)(void *) = nullptr;
+  void *copier = nullptr;             // pinned buffers and threads of host copies
+  void (*copier_free)(void *) = nullptr;
+  lgpu::DevBuf work[4];               // temporaries of ray queries and image operations, kept between calls
   void *scratch = nullptr;            // device address of this GPU's no-allocation scratch array
   std::vector<void *> guides;         // live guiding networks (released with the device)
   void (*guide_orphan)(void *) = nullptr;
+  // Ends a call that used `work`: no kept temporary stays above 128 MiB (a 4K film takes 127).
+  void trim_work() {
+    for (lgpu::DevBuf &b : work)
+      if (b.bytes > (128ull << 20)) b.release();
+  }
 };
 
 struct lgpu_film_s {

@@ -144,7 +144,8 @@ lgpu_status lgpu_film_post(lgpu_film f, const lgpu_post_desc *d, float *rgba, ui
   LGPU_HIP(hipSetDevice(f->dev->device));
   const uint32_t n = f->width * f->height;
   const hipStream_t st = f->dev->stream;
-  DevBuf img, kern, o32, o8;
+  DevBuf kern;
+  DevBuf &img = f->dev->work[0], &o32 = f->dev->work[1], &o8 = f->dev->work[2];
   LGPU_HIP(img.alloc(16ull * n));
   if (conv) LGPU_HIP(kern.upload(d->kernel, 4ull * d->kernel_w * d->kernel_h));
   if (rgba) LGPU_HIP(o32.alloc(16ull * n));
@@ -156,9 +157,9 @@ lgpu_status lgpu_film_post(lgpu_film f, const lgpu_post_desc *d, float *rgba, ui
   hipLaunchKernelGGL(k_post, dim3((n + 255) / 256), dim3(256), 0, st, img.as<float4>(), kern.as<float>(), p,
                      rgba ? o32.as<float4>() : nullptr, rgba8 ? o8.as<uchar4>() : nullptr);
   LGPU_HIP(hipGetLastError());
-  if (rgba) LGPU_HIP(hipMemcpyAsync(rgba, o32.ptr, 16ull * n, hipMemcpyDeviceToHost, st));
-  if (rgba8) LGPU_HIP(hipMemcpyAsync(rgba8, o8.ptr, 4ull * n, hipMemcpyDeviceToHost, st));
-  LGPU_HIP(hipStreamSynchronize(st));
+  if (rgba) LGPU_HIP(CopyToHost(f->dev, rgba, o32.ptr, 16ull * n));
+  if (rgba8) LGPU_HIP(CopyToHost(f->dev, rgba8, o8.ptr, 4ull * n));
+  f->dev->trim_work();
   return LGPU_OK;
 }
 
