@@ -98,3 +98,21 @@ def test_denoise_rejects_bad_arguments(dev):
         a.denoise(abi.denoise_desc(sigma_colour=-1.0))
     with pytest.raises(LambdaError):
         a.denoise(abi.denoise_desc(), normal=b)
+
+
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 70), (64, 16), (65, 17), (130, 33)])
+@pytest.mark.parametrize("iterations", [1, 3, 6])
+def test_denoise_sizes(dev, w, h, iterations):
+    """Image sizes around the filter's tile (64 columns, 4 rows a step apart), steps up to 32 rows."""
+    rng = np.random.default_rng(w + h)
+    films, means = [], []
+    for lo, hi in ((0.0, 2.0), (0.1, 0.9), (0.0, 1.0)):
+        f = gpu.Film(dev, w, h)
+        f.write(rng.uniform(lo, hi, size=(h, w, 3)))
+        films.append(f)
+        means.append(_means(f))
+    d = abi.denoise_desc(iterations=iterations, sigma_colour=0.9, sigma_normal=0.7, sigma_albedo=0.6, demodulate=True)
+    out = gpu.Film(dev, w, h)
+    films[0].denoise(d, albedo=films[1], normal=films[2], out=out)
+    c = oracle.denoise(means[0], d, albedo=means[1], normal=means[2])
+    np.testing.assert_allclose(_means(out), c, rtol=1e-4, atol=1e-6)
