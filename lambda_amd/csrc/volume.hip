@@ -218,7 +218,7 @@ __global__ void k_publish(BounceSlot *slot, BounceSlot *host) {
 
 }  // namespace
 
-void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene *scp, int programs, const RenderParams &rp,
+void LaunchVolFaithful(uint32_t blocks, hipStream_t stream, const DevScene &sc, const RenderParams &rp,
                        PathState ps, SampleState ss, uint32_t n, Queues q, uint32_t *spill, const uint32_t *np,
                        BounceSlot *slot);
 void LaunchVolAdjoint(uint32_t blocks, hipStream_t stream, const DevScene *scp, int programs, const RenderParams &rp,
@@ -231,7 +231,7 @@ uint32_t LaunchShadeVol(uint32_t blocks, hipStream_t stream, const DevScene &sc,
   const int programs = (int)sc.has_programs;
   if (adj || !rp.corrected) {
     if (adj) LaunchVolAdjoint(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, *adj, np, slot);
-    else LaunchVolFaithful(blocks, stream, scp, programs, rp, ps, ss, n, q, spill, np, slot);
+    else LaunchVolFaithful(blocks, stream, sc, rp, ps, ss, n, q, spill, np, slot);
     if (slot) hipLaunchKernelGGL(k_publish, dim3(1), dim3(1), 0, stream, slot, host);
     return 1;
   }

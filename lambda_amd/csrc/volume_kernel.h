@@ -1,6 +1,8 @@
 // Volumetric shade kernel (volume.hip describes the stage). Its instantiations are spread over
 // volume.hip, volume_faithful.hip and volume_adjoint.hip, which compile in parallel.
 #pragma once
+#include <type_traits>
+
 #include "adjoint.h"
 #include "host.h"
 #include "lights.h"
@@ -17,6 +19,14 @@ namespace lgpu {
 // Faithful: inline, since as written a light sample's pdf depends on the visibility of the one
 // before it. Adjoint: inline, since a vertex's gradients need its visibility at once.
 enum VolMode { kVolSplit, kVolSplitLookup, kVolFaithful, kVolAdjoint };
+
+// The scene record comes through a pointer: a by-value argument whose address reaches out-of-line
+// functions is copied into every lane's scratch. The faithful kernel keeps the by-value record and the
+// default registers it has always been run with.
+template <VolMode kMode>
+using VolScene = std::conditional_t<kMode == kVolFaithful, DevScene, const DevScene *__restrict__>;
+__device__ inline const DevScene &SceneOf(const DevScene &sc) { return sc; }
+__device__ inline const DevScene &SceneOf(const DevScene *sc) { return *sc; }
 
 // Tree index of a light pick, for SampleLi's triangle record.
 __device__ inline uint32_t TreeIdx(uint32_t pick) { return (pick & kTreeBit) ? (pick & ~kTreeBit) : kNone; }
@@ -156,21 +166,19 @@ __device__ inline Spec LdMediumPoint(const DevScene &sc, const MediumRec &M, uin
 }
 
 // kPrograms: what the scene's sockets need (DevScene::has_programs); without program sockets the kernel
-// is compiled without the shader VM. The scene record comes through a pointer: a by-value argument whose
-// address reaches out-of-line functions is copied into every lane's scratch.
+// is compiled without the shader VM.
 // kVolAdjoint: the replay of the adjoint render (RGB, VOLPATH): the same path decisions and radiance
 // as the primal launch, plus the gradient pieces of adjoint.h.
 // np: when set, the item count is read from this device counter (the grid covers an upper bound).
 template <int kPrograms, VolMode kMode>
-__global__ void __launch_bounds__(kBlock, kMode == kVolSplit ? 4 : 2)
-    k_shade_vol(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
+__global__ void __launch_bounds__(kBlock, kMode == kVolSplit ? 4 : 2) k_shade_vol(VolScene<kMode> scene, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
                 const uint32_t *np, Queues q, uint32_t *spillBase, AdjRefs ar, BounceSlot *slot) {
   if (slot) Stamp(&slot->shade);
   constexpr bool kAdjoint = kMode == kVolAdjoint;
   constexpr bool kSplit = kMode == kVolSplit || kMode == kVolSplitLookup;  // rays resolved by k_vol_light, k_vol_shadow
   constexpr bool kTraces = kMode != kVolSplit;
   constexpr bool corrected = kMode != kVolFaithful;
-  const DevScene &sc = *scp;
+  const DevScene &sc = SceneOf(scene);
   __shared__ uint32_t stk[kTraces ? kLdsStack : 1][kBlock];
   __shared__ TreeImp treeLds[kTreeLds];
   __shared__ uint32_t pushLds[kBlock / 64 + 1];
