@@ -776,12 +776,11 @@ static void LaunchShade(bool corrected, int programs, const GuideRefs *gr, uint3
 }
 
 // ---------------------------------------------------------------- batched renders (batch.hip)
-// Counter slots of one job's chunk: slot 0 = the camera's path count, the rest cleared (inside a
-// captured graph, where memset nodes are avoided).
+// Counter slots of one job's chunk: slot 0 = the camera's path count, the rest cleared.
 __global__ void k_batch_init(uint32_t *ctr, uint32_t words, uint32_t n) {
   for (uint32_t k = threadIdx.x; k < words; k += blockDim.x) ctr[k] = k == 0 ? n : 0u;
 }
-// Paths still queued after a chunk's last captured iteration (must stay 0).
+// Paths still queued after a chunk's last issued iteration (must stay 0).
 __global__ void k_batch_trunc(const uint32_t *cnt, unsigned long long *acc) {
   if (threadIdx.x == 0 && *cnt) atomicAdd(acc, (unsigned long long)*cnt);
 }

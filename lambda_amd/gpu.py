@@ -449,7 +449,7 @@ def render(desc):
 
 
 def render_batch(descs, path_capacity=0, autotune=False, branches=0, max_iterations=0):
-    """Renders every job (render_desc) together from one path pool, one hipGraph per chunk."""
+    """Renders every job (render_desc) together from one path pool, the jobs on streams side by side."""
     arr = (abi.RenderDesc * len(descs))(*descs)
     o = abi.BatchOptions()
     o.path_capacity = path_capacity
