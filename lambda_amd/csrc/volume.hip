@@ -104,8 +104,9 @@ __device__ inline uint32_t BlockGather(bool take, uint32_t *cnt, uint16_t *list,
 // Step 1 for the block's paths that reach a light or cross a boundary: the light reached by the
 // previous vertex's sampled direction, added to the sample's radiance. Paths whose lookup has to walk
 // on through pass-through surfaces come first, so the walking waves are full.
+// Five waves per SIMD, here and in k_vol_shadow: media workload 15.9 ms at four, 15.4 at five and at six.
 template <int kPrograms>
-__global__ void __launch_bounds__(kBlock, 4)
+__global__ void __launch_bounds__(kBlock, 5)
     k_vol_light(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
                 const uint32_t *np, uint32_t *spillBase, BounceSlot *slot) {
   if (slot) Stamp(&slot->shade);
@@ -168,7 +169,7 @@ __global__ void __launch_bounds__(kBlock, 4)
 
 // The visibility rays of the block's vertices (VolRays), slot by slot: a slot's rays are gathered
 // into full waves, and a path's second ray adds to its radiance after its first.
-__global__ void __launch_bounds__(kBlock, 4)
+__global__ void __launch_bounds__(kBlock, 5)
     k_vol_shadow(const DevScene *__restrict__ scp, RenderParams rp, PathState ps, SampleState ss, uint32_t n,
                  const uint32_t *np, uint32_t *spillBase, int slots, BounceSlot *slot, BounceSlot *host) {
   if (slot && blockIdx.x == 0 && threadIdx.x == 0) Publish(slot, host);  // closes the bounce
