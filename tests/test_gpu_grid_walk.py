@@ -1,5 +1,5 @@
 """Grid media whose walks end inside, at and past a group of voxels stepped ahead (one voxel, fewer than a
-group along an axis, many), against the CPU checker path by path (1e-4 relative + 1e-6, 99.9 % of paths as
+group along an axis, many), against the CPU oracle path by path (1e-4 relative + 1e-6, 99.9 % of paths as
 in the media parity tests)."""
 import numpy as np
 import pytest

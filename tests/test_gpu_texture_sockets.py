@@ -1,4 +1,4 @@
-"""Sockets that are one texture lookup (no shader program), in every form they take, against the CPU checker
+"""Sockets that are one texture lookup (no shader program), in every form they take, against the CPU oracle
 path by path (1e-4 relative + 1e-6, 99.9 % of paths as in the media parity tests): textures of 1, 3 and 4
 channels read as a spectrum, a broadcast channel, a real and a roughness."""
 import numpy as np

@@ -1,4 +1,4 @@
-"""The volumetric shade stage at the edges of its 256-path blocks, against the CPU checker path by path
+"""The volumetric shade stage at the edges of its 256-path blocks, against the CPU oracle path by path
 (1e-4 relative + 1e-6, 99.9 % of paths as in the media parity tests)."""
 import numpy as np
 import pytest

@@ -1,5 +1,5 @@
 """The volumetric stage's rays in kernels of their own, one scene for each way a ray can be resolved,
-against the CPU checker path by path (1e-4 relative + 1e-6, 99.9 % of paths as in the media parity tests)."""
+against the CPU oracle path by path (1e-4 relative + 1e-6, 99.9 % of paths as in the media parity tests)."""
 import math
 
 import numpy as np
