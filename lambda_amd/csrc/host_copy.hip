@@ -17,8 +17,9 @@ namespace lgpu {
 namespace {
 
 constexpr size_t kChunk = 1u << 20;    // bytes per transfer
-constexpr int kChunks = 16;            // pinned buffers: 16 MiB per device object
 constexpr int kCopyThreads = 6;
+constexpr int kOwn = 2;                // pinned buffers of a thread: one is copied while the other is on the bus
+constexpr int kChunks = kOwn * kCopyThreads;  // 12 MiB per device object
 constexpr size_t kDirect = 1u << 20;   // copies up to this size: the runtime's copy (chunking gains nothing)
 
 struct HostCopier {
@@ -49,9 +50,8 @@ struct HostCopier {
       if (e) (void)hipEventDestroy(e);
     if (pinned) (void)hipHostFree(pinned);
   }
-  // Each thread owns kChunks / kCopyThreads buffers and takes the next chunk of the job for each.
+  // Each thread owns kOwn buffers and takes the next chunk of the job for each.
   void Work(int id) {
-    constexpr int kOwn = kChunks / kCopyThreads;
     const size_t count = (bytes + kChunk - 1) / kChunk;
     size_t at[kOwn];
     bool full[kOwn] = {};
