@@ -12,3 +12,26 @@ for _ in range(4): f.read()
 held = H.host_hip_pinned() - before
 assert held == 12 * MB, held
 """)
+
+
+def test_small_copies_wait_for_no_other_thread(host_hip):
+    """A read of two chunks (1.5 MiB) is done by the calling thread; longer ones give what was written,
+    whichever thread takes which chunk."""
+    host_hip("""
+f = gpu.Film(dev, 256, 256)
+a = np.random.default_rng(0).random((256, 256, 3))
+f.write(a)
+copies()
+me = threading.get_native_id()
+for _ in range(20):
+    got, cnt = f.read()
+    assert (got == a).all()
+    big = [c for c in copies() if c[1] > 512 * 1024]
+    assert big and all(c[3] == me for c in big), big
+for w, h in ((256, 300), (512, 341), (1021, 1531)):
+    f = gpu.Film(dev, w, h)
+    a = np.random.default_rng(1).random((h, w, 3))
+    f.write(a)
+    for _ in range(20):
+        assert (f.read()[0] == a).all()
+""")
