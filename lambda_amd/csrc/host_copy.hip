@@ -23,7 +23,11 @@ constexpr size_t kChunk = 1u << 20;    // bytes per transfer
 constexpr int kCopyThreads = 6;        // the caller and five helpers
 constexpr int kOwn = 2;                // pinned buffers of a thread: one is copied while the other is on the bus
 constexpr int kChunks = kOwn * kCopyThreads;  // 12 MiB per device object
-constexpr size_t kDirect = 1u << 20;   // copies up to this size (one chunk): the runtime's copy
+// Copies up to these sizes are the runtime's: one chunk to the host; below 32 MiB to the device, where the
+// source's pages are there and the runtime copies from them in place (film writes of 2, 8 and 24 MiB: the
+// runtime 94, 310 and 850 us, chunks 117, 415 and 1030; of 30 MiB in a new array 1.35 ms and 1.85; from 32
+// MiB both are the same, 1.4 ms, and at 96 MiB the chunks are ahead, 4.2 and 3.95).
+constexpr size_t kDirectToHost = 1u << 20, kDirectToDevice = (32u << 20) - 1;
 
 struct HostCopier {
   uint8_t *pinned = nullptr;
@@ -153,7 +157,7 @@ struct HostCopier {
 
 hipError_t Copy(lgpu_device d, void *host, void *dev, size_t n, bool down) {
   if (!n) return hipSuccess;
-  if (n > kDirect) {
+  if (n > (down ? kDirectToHost : kDirectToDevice)) {
     if (!d->copier) {
       try {
         d->copier = new HostCopier();
