@@ -72,10 +72,10 @@ struct HostLight {
 };
 
 // Film::ToRGBTexture into host memory (4 floats per pixel); the caller holds the device mutex.
-// pinned: rgba is page-locked (copied to directly).
-lgpu_status FilmToRgba(lgpu_film f, float *rgba, bool pinned = false);
-// Copies between a caller's array and device memory, after the work already on the device's stream; the
-// data has arrived on return (host_copy.hip). The caller holds the device mutex.
+lgpu_status FilmToRgba(lgpu_film f, float *rgba);
+// Copies between a caller's array (pageable, page-locked or, as the runtime allows, device memory) and
+// device memory, after the work already on the device's stream; the data has arrived on return
+// (host_copy.hip). The caller holds the device mutex.
 hipError_t CopyToHost(lgpu_device d, void *host, const void *dev, size_t n);
 hipError_t CopyToDevice(lgpu_device d, void *dev, const void *host, size_t n);
 

@@ -29,7 +29,7 @@ __global__ void k_film_rgba(const double *sum, const uint32_t *count, float4 *ou
 }  // namespace
 
 // Film::ToRGBTexture into host memory (rgba: 4 floats per pixel). The caller holds the device mutex.
-lgpu_status FilmToRgba(lgpu_film f, float *rgba, bool pinned) {
+lgpu_status FilmToRgba(lgpu_film f, float *rgba) {
   const uint32_t n = f->width * f->height;
   LGPU_HIP(hipSetDevice(f->dev->device));
   DevBuf &out = f->dev->work[0];
@@ -37,12 +37,7 @@ lgpu_status FilmToRgba(lgpu_film f, float *rgba, bool pinned) {
   hipLaunchKernelGGL(k_film_rgba, dim3((n + 255) / 256), dim3(256), 0, f->dev->stream, f->sum.as<double>(),
                      f->count.as<uint32_t>(), out.as<float4>(), n);
   LGPU_HIP(hipGetLastError());
-  if (pinned) {
-    LGPU_HIP(hipMemcpyAsync(rgba, out.ptr, 16ull * n, hipMemcpyDeviceToHost, f->dev->stream));
-    LGPU_HIP(hipStreamSynchronize(f->dev->stream));
-  } else {
-    LGPU_HIP(CopyToHost(f->dev, rgba, out.ptr, 16ull * n));
-  }
+  LGPU_HIP(CopyToHost(f->dev, rgba, out.ptr, 16ull * n));
   f->dev->trim_work();
   return LGPU_OK;
 }
@@ -79,7 +74,7 @@ struct lgpu_progressive_s {
       lgpu_status st = lgpu_render(&d, nullptr);  // ProgressiveRender::RunPass: every tile, one increment
       if (st == LGPU_OK) {
         std::lock_guard<std::mutex> lk(f->dev->mu);
-        st = FilmToRgba(f, buf[front ^ 1], true);  // ProgressiveRender::UpdateOutputTexture
+        st = FilmToRgba(f, buf[front ^ 1]);  // ProgressiveRender::UpdateOutputTexture
       }
       if (st != LGPU_OK) { Record(st); break; }
       ++passes;

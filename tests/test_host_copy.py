@@ -50,3 +50,34 @@ for w, h, chunked in ((256, 250, False), (1024, 1024, False), (1280, 1024, False
     assert len(sums) == (0 if chunked else 1), (w, h, up)
     assert (f.read()[0] == a).all()
 """)
+
+
+def test_page_locked_and_device_memory_is_copied_directly(host_hip):
+    """A page-locked array, or device memory in the place of a host array, takes one copy of the whole
+    range, in both directions and from any place inside the allocation; an ordinary array goes by chunks."""
+    host_hip("""
+H.hipHostMalloc.argtypes = [C.c_void_p, C.c_size_t, C.c_uint]
+H.hipMalloc.argtypes = [C.c_void_p, C.c_size_t]
+L = gpu.lib()
+w, h = 1600, 1100
+n = 24 * w * h
+f = gpu.Film(dev, w, h)
+a = np.random.default_rng(3).random((h, w, 3))
+for kind in ("pinned", "device"):
+    p = C.c_void_p()
+    assert (H.hipHostMalloc(C.byref(p), n + 4096, 0) if kind == "pinned" else H.hipMalloc(C.byref(p), n + 4096)) == 0
+    at = p.value + 264
+    C.memmove(at, a.ctypes.data, n)
+    cnt = np.ones((h, w), dtype=np.uint32)
+    copies()
+    assert L.lgpu_film_write(f.h, at, cnt.ctypes.data) == 0
+    assert [c for c in copies() if c[0] == at and c[1] == n and c[2] == 1], kind
+    C.memset(at, 0, n)
+    assert L.lgpu_film_read(f.h, at, None) == 0
+    c = copies()
+    assert len(c) == 1 and c[0][0] == at and c[0][1] == n, (kind, c)
+    assert C.string_at(at, n) == a.tobytes()
+copies()
+f.read()
+assert sum(c[1] == MB for c in copies()) == n // MB + 4 * w * h // MB
+""")
