@@ -29,18 +29,21 @@ constexpr uint32_t kCtrStride = 32;  // words between a job's counters of two bo
 
 // Path state of a batch's jobs, kept on the device object between calls while it is small (some twenty
 // allocations and releases a call: 15.1 ms with them, 9.0 ms without, for eight scenes of 48 to 384
-// pixels a side). A pool above kKeepBytes is given back at the end of the call.
+// pixels a side). A pool above kKeepBytes is given back at the end of the call, and a call that fails gives
+// back all of it: its buffers may have grown to a size that the next one cannot afford beside its own.
 constexpr uint64_t kKeepBytes = 1ull << 30;
 struct BatchPool {
   DevBuf st[2][9], L, pix, lam, shadow, spill, scenes, ctr, trunc;
-  void trim() {
-    uint64_t b = L.bytes + pix.bytes + lam.bytes + shadow.bytes + spill.bytes;
+  void end(bool ok) {
+    DevBuf *rest[] = {&L, &pix, &lam, &shadow, &spill, &scenes, &ctr, &trunc};
+    uint64_t b = 0;
     for (const auto &row : st)
       for (const DevBuf &x : row) b += x.bytes;
-    if (b <= kKeepBytes) return;
+    for (const DevBuf *x : rest) b += x->bytes;
+    if (ok && b <= kKeepBytes) return;
     for (auto &row : st)
       for (DevBuf &x : row) x.release();
-    for (DevBuf *x : {&L, &pix, &lam, &shadow, &spill}) x->release();
+    for (DevBuf *x : rest) x->release();
   }
 };
 
@@ -137,6 +140,11 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
   Branches &br = BranchesOf(dev);
   { lgpu_status s = br.init(); if (s != LGPU_OK) return s; }
   BatchPool &P = br.pool;
+  struct Use {  // every way out of the call, with no kernel left on the streams
+    BatchPool &pool;
+    bool ok = false;
+    ~Use() { pool.end(ok); }
+  } use{P};
   for (int b = 0; b < 2; ++b)
     for (int k = 0; k < 9; ++k) LGPU_HIP(P.st[b][k].alloc(16 * N));
   LGPU_HIP(P.L.alloc(16 * N));
@@ -253,7 +261,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
   if (se != hipSuccess) return Fail(LGPU_ERR_HIP, std::string("render_batch: ") + hipGetErrorString(se));
   unsigned long long trunc = 0;
   LGPU_HIP(hipMemcpy(&trunc, P.trunc.ptr, 8, hipMemcpyDeviceToHost));
-  P.trim();
+  use.ok = true;
   if (trunc)
     return Fail(LGPU_ERR_STATE, "render_batch: " + std::to_string(trunc) +
                                     " paths outlived the captured iterations (raise max_iterations)");

@@ -1,0 +1,53 @@
+"""Device memory that the library keeps between calls, and what a failed call gives back. Run on the CPU
+(tests/host_hip.py) with a budget of device memory, so that allocations fail part way."""
+from tests.host_hip import host_hip  # noqa: F401
+
+GIB = 1 << 30
+
+BATCH = """
+GIB = 1 << 30
+def job(side, spp, s, cap=0):
+    f = gpu.Film(dev, side, side)
+    return gpu.render_desc(s, f, scene.cornell_camera(side, side), 0, spp, max_bounces=4, estimator=abi.ESTIMATOR_CORRECTED,
+                           capacity=cap), f
+s = gpu.Scene(dev)
+scene.cornell_box().push(s, abi.LIGHTS_TREE)
+small, fs = job(64, 4, s)
+large, fl = job(1024, 64, s)          # 2^26 paths, some 22 GiB
+fits, ff = job(1024, 8, s)            # 2^23 paths, 2.8 GiB
+"""
+
+
+def test_failed_batch_gives_its_pool_back(host_hip):
+    """A batch that runs out of device memory keeps nothing of its pool: what fits afterwards is what fitted
+    before, a small batch and a render among it."""
+    host_hip(BATCH + """
+before = live()
+H.host_hip_budget(before + 7 * GIB // 2)
+try:
+    gpu.render_batch([large], path_capacity=1 << 26)
+    raise SystemExit("the large batch fitted")
+except gpu.LambdaError as e:
+    assert "memory" in str(e), e
+assert live() - before < 1 * MB, (live() - before) / MB
+gpu.render_batch([small])
+assert live() - before < 64 * MB, (live() - before) / MB
+gpu.render(fits)
+""")
+
+
+def test_batch_pool_is_kept_up_to_its_bound(host_hip):
+    """The pool of a small batch stays (no allocation in a second call); all of a pool above 1 GiB is given
+    back, counters of many iterations included."""
+    host_hip(BATCH + """
+before = live()
+gpu.render_batch([small])
+kept = live() - before
+assert 0 < kept < 64 * MB
+gpu.render_batch([small])
+assert live() - before == kept
+gpu.render_batch([fits])
+assert live() - before < 1 * MB, (live() - before) / MB
+gpu.render_batch([small], max_iterations=(GIB + GIB // 16) // 128)
+assert live() - before < 1 * MB, (live() - before) / MB
+""")
