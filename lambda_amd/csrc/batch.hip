@@ -25,7 +25,7 @@ namespace lgpu {
 namespace {
 
 constexpr uint32_t kMaxBranches = 16;
-constexpr uint32_t kCtrStride = 32;  // words between a job's counters of two bounces: a 128-byte line each (BounceSlot)
+constexpr uint64_t kCtrStride = 32;  // words between a job's counters of two bounces: a 128-byte line each (BounceSlot)
 
 // Path state of a batch's jobs, kept on the device object between calls while it is small (some twenty
 // allocations and releases a call: 15.1 ms with them, 9.0 ms without, for eight scenes of 48 to 384
@@ -123,7 +123,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
   }
   // bounce iterations per chunk: bounces plus pass-through crossings (which do not count as bounces)
   const uint32_t iters = iterations ? iterations : 2 * maxB + 8;
-  const uint32_t ctrWords = kCtrStride * (iters + 1);
+  const uint64_t ctrWords = kCtrStride * ((uint64_t)iters + 1);  // no iteration count reaches past its job's
   // segments in proportion to the jobs' paths, at least one block each
   std::vector<uint32_t> cap(J);
   std::vector<uint64_t> off(J + 1, 0), spillOff(J + 1, 0);
@@ -156,7 +156,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
   for (uint32_t j = 0; j < J; ++j) scenes[j] = d[j].scene->dsc;
   LGPU_HIP(P.scenes.alloc(sizeof(DevScene) * J));
   LGPU_HIP(hipMemcpy(P.scenes.ptr, scenes.data(), sizeof(DevScene) * J, hipMemcpyHostToDevice));
-  LGPU_HIP(P.ctr.alloc(4ull * ctrWords * J));
+  LGPU_HIP(P.ctr.alloc(4 * ctrWords * J));
   LGPU_HIP(P.trunc.alloc(8));
   LGPU_HIP(hipMemset(P.trunc.ptr, 0, 8));
   LGPU_HIP(hipDeviceSynchronize());
@@ -188,7 +188,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
     b.ss.lambda0 = P.lam.as<float>() + off[j];
     b.shadow = P.shadow.as<ShadowRay>() + off[j];
     b.spill = P.spill.as<uint32_t>() + spillOff[j];
-    b.ctr = P.ctr.as<uint32_t>() + (size_t)ctrWords * j;
+    b.ctr = P.ctr.as<uint32_t>() + ctrWords * j;
     b.scp = P.scenes.as<DevScene>() + j;
     b.path = d[j].integrator == LGPU_INTEGRATOR_PATH;
     b.programs = (int)scenes[j].has_programs;
@@ -219,7 +219,7 @@ lgpu_status RunBatch(const lgpu_render_desc *d, uint32_t count, uint64_t capacit
           const Job &b = jobs[j];
           hipStream_t s = br.s[j % branches];
           const uint32_t cur = it & 1u;
-          uint32_t *cin = b.ctr + kCtrStride * it, *cout = b.ctr + kCtrStride * (it + 1);
+          uint32_t *cin = b.ctr + kCtrStride * it, *cout = cin + kCtrStride;
           BatchLaunchExtend(s, scenes[j], b.ps[cur], n[j], cin, b.spill);
           const Queues q{b.ps[cur ^ 1u], b.shadow, cout};
           if (b.path) {

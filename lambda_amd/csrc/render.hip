@@ -777,14 +777,14 @@ static void LaunchShade(bool corrected, int programs, const GuideRefs *gr, uint3
 
 // ---------------------------------------------------------------- batched renders (batch.hip)
 // Counter slots of one job's chunk: slot 0 = the camera's path count, the rest cleared.
-__global__ void k_batch_init(uint32_t *ctr, uint32_t words, uint32_t n) {
-  for (uint32_t k = threadIdx.x; k < words; k += blockDim.x) ctr[k] = k == 0 ? n : 0u;
+__global__ void k_batch_init(uint32_t *ctr, uint64_t words, uint32_t n) {
+  for (uint64_t k = threadIdx.x; k < words; k += blockDim.x) ctr[k] = k == 0 ? n : 0u;
 }
 // Paths still queued after a chunk's last issued iteration (must stay 0).
 __global__ void k_batch_trunc(const uint32_t *cnt, unsigned long long *acc) {
   if (threadIdx.x == 0 && *cnt) atomicAdd(acc, (unsigned long long)*cnt);
 }
-void BatchLaunchInit(hipStream_t s, uint32_t *ctr, uint32_t words, uint32_t n) {
+void BatchLaunchInit(hipStream_t s, uint32_t *ctr, uint64_t words, uint32_t n) {
   hipLaunchKernelGGL(k_batch_init, dim3(1), dim3(64), 0, s, ctr, words, n);
 }
 void BatchLaunchTrunc(hipStream_t s, const uint32_t *cnt, unsigned long long *acc) {

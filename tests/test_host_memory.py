@@ -51,3 +51,16 @@ assert live() - before < 1 * MB, (live() - before) / MB
 gpu.render_batch([small], max_iterations=(GIB + GIB // 16) // 128)
 assert live() - before < 1 * MB, (live() - before) / MB
 """)
+
+
+def test_counters_of_any_iteration_count_are_allocated(host_hip):
+    """A job's queue counters take 128 bytes an iteration: 2^27 iterations do not fit 4 GiB and are refused
+    for that (a 32-bit word count would wrap to a few bytes and the kernels would count past them)."""
+    host_hip(BATCH + """
+try:
+    gpu.render_batch([small], max_iterations=1 << 27)
+    raise SystemExit("not refused")
+except gpu.LambdaError as e:
+    assert "memory" in str(e), e
+gpu.render_batch([small])
+""")
