@@ -142,6 +142,7 @@ lgpu_status lgpu_film_denoise(lgpu_film colour, lgpu_film albedo, lgpu_film norm
   LGPU_HIP(hipSetDevice(colour->dev->device));
   (void)hipGetLastError();
   const hipStream_t st = colour->dev->stream;
+  WorkUse use{colour->dev};
   DevBuf &ca = colour->dev->work[0], &cb = colour->dev->work[1], &ab = colour->dev->work[2], &nb = colour->dev->work[3];
   LGPU_HIP(ca.alloc(16ull * n));
   LGPU_HIP(cb.alloc(16ull * n));
@@ -176,9 +177,9 @@ lgpu_status lgpu_film_denoise(lgpu_film colour, lgpu_film albedo, lgpu_film norm
   }
   const hipError_t le = hipGetLastError();
   const hipError_t se = hipStreamSynchronize(st);  // before the buffers are used by another call
-  colour->dev->trim_work();
   LGPU_HIP(le);
   LGPU_HIP(se);
+  use.ok = true;
   return LGPU_OK;
 }
 

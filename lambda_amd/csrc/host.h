@@ -92,16 +92,26 @@ struct lgpu_device_s {
   void (*batch_free)(void *) = nullptr;
   void *copier = nullptr;             // pinned buffers and threads of host copies
   void (*copier_free)(void *) = nullptr;
-  lgpu::DevBuf work[4];               // temporaries of ray queries and image operations, kept between calls
+  lgpu::DevBuf work[4];               // temporaries of ray queries and image operations, kept between calls (WorkUse)
   void *scratch = nullptr;            // device address of this GPU's no-allocation scratch array
   std::vector<void *> guides;         // live guiding networks (released with the device)
   void (*guide_orphan)(void *) = nullptr;
-  // Ends a call that used `work`: no kept temporary stays above 128 MiB (a 4K film takes 127).
-  void trim_work() {
-    for (lgpu::DevBuf &b : work)
-      if (b.bytes > (128ull << 20)) b.release();
+};
+
+namespace lgpu {
+// A call's use of a device's `work`, ended on every way out of it: no kept temporary stays above 128 MiB (a
+// 4K film takes 127), and a call that fails gives all of them back, since what it obtained may be what the
+// next one lacks. The caller holds the device mutex.
+struct WorkUse {
+  lgpu_device dev;
+  bool ok = false;
+  ~WorkUse() {
+    if (!ok) (void)hipStreamSynchronize(dev->stream);
+    for (DevBuf &b : dev->work)
+      if (!ok || b.bytes > (128ull << 20)) b.release();
   }
 };
+}  // namespace lgpu
 
 struct lgpu_film_s {
   lgpu_device dev = nullptr;

@@ -145,6 +145,7 @@ lgpu_status lgpu_film_post(lgpu_film f, const lgpu_post_desc *d, float *rgba, ui
   const uint32_t n = f->width * f->height;
   const hipStream_t st = f->dev->stream;
   DevBuf kern;
+  WorkUse use{f->dev};
   DevBuf &img = f->dev->work[0], &o32 = f->dev->work[1], &o8 = f->dev->work[2];
   LGPU_HIP(img.alloc(16ull * n));
   if (conv) LGPU_HIP(kern.upload(d->kernel, 4ull * d->kernel_w * d->kernel_h));
@@ -159,7 +160,7 @@ lgpu_status lgpu_film_post(lgpu_film f, const lgpu_post_desc *d, float *rgba, ui
   LGPU_HIP(hipGetLastError());
   if (rgba) LGPU_HIP(CopyToHost(f->dev, rgba, o32.ptr, 16ull * n));
   if (rgba8) LGPU_HIP(CopyToHost(f->dev, rgba8, o8.ptr, 4ull * n));
-  f->dev->trim_work();
+  use.ok = true;
   return LGPU_OK;
 }
 

@@ -32,13 +32,14 @@ __global__ void k_film_rgba(const double *sum, const uint32_t *count, float4 *ou
 lgpu_status FilmToRgba(lgpu_film f, float *rgba) {
   const uint32_t n = f->width * f->height;
   LGPU_HIP(hipSetDevice(f->dev->device));
+  WorkUse use{f->dev};
   DevBuf &out = f->dev->work[0];
   LGPU_HIP(out.alloc(16ull * n));
   hipLaunchKernelGGL(k_film_rgba, dim3((n + 255) / 256), dim3(256), 0, f->dev->stream, f->sum.as<double>(),
                      f->count.as<uint32_t>(), out.as<float4>(), n);
   LGPU_HIP(hipGetLastError());
   LGPU_HIP(CopyToHost(f->dev, rgba, out.ptr, 16ull * n));
-  f->dev->trim_work();
+  use.ok = true;
   return LGPU_OK;
 }
 

@@ -1427,6 +1427,7 @@ static lgpu_status Query(lgpu_scene s, uint32_t n, const float *rays, uint32_t *
   std::lock_guard<std::mutex> lk(s->dev->mu);
   LGPU_HIP(hipSetDevice(s->dev->device));
   (void)hipGetLastError();
+  WorkUse use{s->dev};
   DevBuf &dr = s->dev->work[0], &dh = s->dev->work[1], &dsp = s->dev->work[2];
   LGPU_HIP(dr.alloc(32ull * n));
   LGPU_HIP(CopyToDevice(s->dev, dr.ptr, rays, 32ull * n));
@@ -1434,10 +1435,9 @@ static lgpu_status Query(lgpu_scene s, uint32_t n, const float *rays, uint32_t *
   LGPU_HIP(dsp.alloc(std::max<size_t>(256, 4ull * s->dsc.spill_words * n)));
   hipLaunchKernelGGL(k_query, dim3(Blocks(n)), dim3(kBlock), 0, s->dev->stream, s->dsc, dr.as<float4>(), n,
                      occ ? nullptr : dh.as<uint4>(), occ ? dh.as<uint32_t>() : nullptr, dsp.as<uint32_t>());
-  const hipError_t le = hipGetLastError();
-  LGPU_HIP(le);
+  LGPU_HIP(hipGetLastError());
   LGPU_HIP(CopyToHost(s->dev, occ ? (void *)occ : (void *)hits, dh.ptr, occ ? 4ull * n : 16ull * n));
-  s->dev->trim_work();
+  use.ok = true;
   return LGPU_OK;
 }
 extern "C" lgpu_status lgpu_intersect(lgpu_scene s, uint32_t n, const float *rays, uint32_t *hits) {

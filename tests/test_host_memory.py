@@ -64,3 +64,56 @@ except gpu.LambdaError as e:
     assert "memory" in str(e), e
 gpu.render_batch([small])
 """)
+
+
+FILM = """
+def film(w, h):
+    f = gpu.Film(dev, w, h)
+    return f
+def fails(call):
+    try:
+        call()
+    except gpu.LambdaError as e:
+        assert "memory" in str(e), e
+    else:
+        raise SystemExit("fitted")
+"""
+
+
+def test_failed_film_operations_keep_no_temporaries(host_hip):
+    """Denoising, post-processing and reading an image of a film whose temporaries do not fit: what was
+    obtained is given back, and the same operations on a small film go through."""
+    host_hip(FILM + """
+big, small = film(3600, 3000), film(64, 48)   # 165 MiB an RGBA temporary
+big.read_rgba(), big.read()                   # the copier's buffers
+before = live()
+post, _ = abi.post_desc()
+for call, temporaries in ((lambda f: f.denoise(abi.denoise_desc(), albedo=f, normal=f), 3.5), (lambda f: f.post(post), 1.5)):
+    H.host_hip_budget(before + int(temporaries * 165 * MB))
+    fails(lambda: call(big))
+    assert live() == before, (live() - before) / MB
+    call(small)
+    assert live() - before < 1 * MB
+    H.host_hip_budget(before + 1000 * MB)
+    call(big)
+    assert live() - before < 50 * MB, (live() - before) / MB  # the 8-bit image, below the bound
+    before = live()
+""")
+
+
+def test_failed_ray_batch_keeps_no_temporaries(host_hip):
+    """A ray batch whose hit records do not fit beside the rays."""
+    host_hip(FILM + """
+s = gpu.Scene(dev)
+scene.cornell_box().push(s, abi.LIGHTS_TREE)
+rays = np.zeros((5 << 20, 8), dtype=np.float32)     # 160 MiB of rays, 80 of hits
+s.intersect(rays[:1000])
+before = live()
+H.host_hip_budget(before + 200 * MB)
+fails(lambda: s.intersect(rays))
+assert live() - before < 1 * MB, (live() - before) / MB
+s.intersect(rays[:1000])
+H.host_hip_budget(before + 400 * MB)
+s.intersect(rays)
+assert live() - before < 100 * MB
+""")
