@@ -680,9 +680,8 @@ __device__ inline void SampleRGB(const RenderParams &rp, float4 Lf, float l0, do
 // Per-sample film update for list-mode waves (any pixel may repeat): FP64 atomics, or the raw
 // per-sample record when `out` is set.
 __global__ void __launch_bounds__(kBlock) k_accumulate(RenderParams rp, SampleState ss, uint32_t n, double *film,
-                                                       uint32_t *counts, float *out, unsigned long long *host) {
+                                                       uint32_t *counts, float *out) {
   const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (host && i == 0) *host = wall_clock64();
   if (i >= n) return;
   const float4 Lf = ss.L[i];
   const float l0 = ss.lambda0[i];
@@ -708,9 +707,8 @@ __global__ void __launch_bounds__(kBlock) k_accumulate(RenderParams rp, SampleSt
 // pixel's samples of the wave in sample order and updates its film entry once: each pixel has
 // one owner per launch (t < min(n, npx)), so no atomics are needed and the sum order is fixed.
 __global__ void __launch_bounds__(kBlock) k_accumulate_px(RenderParams rp, SampleState ss, uint32_t n, uint32_t npx,
-                                                          double *film, uint32_t *counts, unsigned long long *host) {
+                                                          double *film, uint32_t *counts) {
   const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-  if (host && t == 0) *host = wall_clock64();
   if (t >= n || t >= npx) return;
   const uint32_t px = ss.pixel[t];
   double *f = film + 3 * (size_t)px;
@@ -812,8 +810,7 @@ void BatchLaunchShadow(hipStream_t s, const DevScene &dsc, const SampleState &ss
 void BatchLaunchAccumulate(hipStream_t s, const RenderParams &rp, const SampleState &ss, uint32_t n, uint32_t npx,
                            double *film, uint32_t *counts) {
   const uint32_t m = n < npx ? n : npx;
-  hipLaunchKernelGGL(k_accumulate_px, dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ss, n, npx, film, counts,
-                     nullptr);
+  hipLaunchKernelGGL(k_accumulate_px, dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rp, ss, n, npx, film, counts);
 }
 
 // Guiding hooks (guide.hip).
@@ -842,7 +839,7 @@ struct Wave {
   unsigned long long *tcount_p = nullptr;
   DevScene *scene_p = nullptr;
   // pipelined path loop: device slots, their pinned host copies, an event per slot (its bounce is
-  // done), and the device clock at a wave's start and at its film update (pinned)
+  // done), and the device clock at a wave's start (pinned)
   static constexpr int kSlots = 4;
   BounceSlot *hring = nullptr;
   unsigned long long *hwave = nullptr;
@@ -1046,12 +1043,21 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
   if (countTrav) LGPU_HIP(hipMemsetAsync(W.tcount_p, 0, 40, stream));
   lgpu_guide G = d->guide;
   GuideRefs gref{};
-  // pipelined loops: a bounce's last stage lasts until the next stamp
+  // pipelined loops: a bounce's last stage lasts until the next bounce begins. A wave's last one: until the
+  // empty bounce issued behind it does (slot `tail`), read before a later wave takes the slot again; neither
+  // the empty bounces nor what follows the wave (a guide's training, the film update) are in it.
   double *open = nullptr;
   unsigned long long openAt = 0;
+  int tail = 0;
   auto CloseStage = [&](unsigned long long at) {
     if (open) *open += W.ms_per_tick * (double)(at - openAt);
     open = nullptr;
+  };
+  auto CloseTail = [&]() -> hipError_t {
+    if (!open) return hipSuccess;
+    const hipError_t e = hipEventSynchronize(W.pev[tail]);
+    if (e == hipSuccess) CloseStage(W.hring[tail].extend);
+    return e;
   };
   for (uint64_t base = 0; base < total; base += cap) {
     const uint32_t n = (uint32_t)std::min<uint64_t>(cap, total - base);
@@ -1092,6 +1098,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
       static_assert(kLag < Wave::kSlots, "a counter slot is reused only after its bounce retired");
       uint32_t ub = n, live = n, issued = 0, retired = 0;
       bool done = false;
+      LGPU_HIP(CloseTail());  // the camera stage is queued behind it: the GPU does not wait
       while (!done) {
         if (issued < maxIter && issued - retired < (uint32_t)kLag) {
           const int sl = (int)(issued % Wave::kSlots), prev = (int)((issued + Wave::kSlots - 1) % Wave::kSlots);
@@ -1136,14 +1143,14 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         const int sl = (int)(retired % Wave::kSlots);
         LGPU_HIP(hipEventSynchronize(W.pev[sl]));
         const BounceSlot b = W.hring[sl];
-        if (retired == 0) S.ms_camera += W.ms_per_tick * (double)(b.extend - W.hwave[0]);
+        if (retired == 0) S.ms_camera += W.ms_per_tick * (double)(b.extend - *W.hwave);
         ++retired;
         const uint32_t c0 = b.next, c1 = b.shadow;
         S.extension_rays += live;
         waveRays += live;
         S.launches_extend++;
         S.launches_shade++;
-        CloseStage(retired == 1 ? W.hwave[1] : b.extend);  // a wave's last one ends where its film update began
+        CloseStage(b.extend);
         S.ms_extend += W.ms_per_tick * (double)((G ? b.infer : b.shade) - b.extend);
         if (G) S.ms_guide_infer += W.ms_per_tick * (double)(b.shade - b.infer);
         if (vol && (ap || !rp.corrected)) {  // one kernel, its end stamped by the publishing one
@@ -1166,6 +1173,8 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         if (c0 == 0) done = true;
       }
       if (!done) return Fail(LGPU_ERR_STATE, "render: path wave did not terminate");
+      if (issued == retired) open = nullptr;  // no bounce behind the last one of the limit
+      tail = (int)(retired % Wave::kSlots);
       if (G) {  // close the wave's records, then train on them before the next wave infers
         const auto tg = std::chrono::steady_clock::now();
         uint32_t recs = 0;
@@ -1233,16 +1242,16 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
     const uint32_t npx = w * h;
     if (!listPix && !out && npx > 0)
       hipLaunchKernelGGL(k_accumulate_px, dim3(Blocks(std::min(n, npx))), dim3(kBlock), 0, stream, rp, W.ss, n, npx, film,
-                         counts, W.hwave ? W.hwave + 1 : nullptr);
+                         counts);
     else
       hipLaunchKernelGGL(k_accumulate, dim3(Blocks(n)), dim3(kBlock), 0, stream, rp, W.ss, n, film, counts,
-                         out ? out + 5 * base : nullptr, W.hwave ? W.hwave + 1 : nullptr);
+                         out ? out + 5 * base : nullptr);
     LGPU_HIP(hipGetLastError());
     }  // rep
     S.waves++;
   }
   LGPU_HIP(hipStreamSynchronize(stream));
-  if (W.hwave) CloseStage(W.hwave[1]);
+  LGPU_HIP(CloseTail());
   if (countTrav) {
     unsigned long long tc[5];
     LGPU_HIP(hipMemcpy(tc, W.tcount_p, 40, hipMemcpyDeviceToHost));

@@ -238,3 +238,29 @@ def test_guiding_reduces_error_on_indirect_light(dev):
         assert rg < 0.9 * rp
     finally:
         g.close()
+
+
+def test_stage_times_of_guided_renders_hold_no_training(dev):
+    """Renders of a few paths, many of which end on a bounce with a shadow ray and no continuation: the
+    stages' times and the training's fit the call's (a stage left open over the training counts it twice)."""
+    sd = scene.cornell_box()
+    s = gpu.Scene(dev)
+    keep = sd.push(s, abi.LIGHTS_TREE)
+    trained = shadows = 0
+    for seed in range(96):
+        g = gpu.Guide(dev, seed=seed, record_capacity=1 << 12)
+        f = gpu.Film(dev, 1, 1)
+        st = gpu.render(gpu.render_desc(s, f, scene.cornell_camera(1, 1), 0, 1, max_bounces=8, min_bounces=8, seed=seed,
+                                        spectral=abi.SPECTRAL_HERO4, estimator=abi.ESTIMATOR_CORRECTED, guide=g,
+                                        guide_train_steps=64))
+        if st.guide_records:
+            trained += 1
+            shadows += st.shadow_rays > 0
+            stages = st.ms_camera + st.ms_extend + st.ms_guide_infer + st.ms_shade + st.ms_shadow
+            assert min(st.ms_camera, st.ms_extend, st.ms_guide_infer, st.ms_shade, st.ms_shadow) >= 0.0
+            assert stages + st.ms_guide_train <= 1.02 * st.ms_total + 0.05, (seed, stages, st.ms_guide_train, st.ms_total)
+        f.close()
+        g.close()
+    assert trained > 10 and shadows > 10, (trained, shadows)
+    del keep
+    s.close()
