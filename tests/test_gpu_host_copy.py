@@ -1,5 +1,6 @@
 """Copies between host arrays and the device at the sizes where their route changes: up to one chunk (1 MiB,
 the runtime's copy), one byte range past it, and more chunks than there are pinned buffers."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -73,3 +74,25 @@ def test_ray_batches(dev, n):
         np.testing.assert_array_equal(occ[a:a + 1000], s.occluded(rays[a:a + 1000]))
     del keep
     s.close()
+
+
+@pytest.mark.parametrize("w,h", [(209, 209), (210, 210), (1021, 1531)])
+def test_film_round_trip_through_page_locked_arrays(dev, w, h):
+    n = 3 * w * h
+    L = gpu.lib()  # its handle gives the HIP runtime's own functions too
+    L.hipHostMalloc.argtypes = [C.c_void_p, C.c_size_t, C.c_uint]
+    L.hipHostFree.argtypes = [C.c_void_p]
+    p = C.c_void_p()
+    assert L.hipHostMalloc(C.byref(p), 8 * (2 * n + 5), 0) == 0
+    mem = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), (2 * n + 5,))
+    up, down = mem[5:5 + n], mem[5 + n:]
+    up[:] = np.random.default_rng(n).random(n)
+    down[:] = 0.0
+    f = gpu.Film(dev, w, h)
+    cnt = np.ones((h, w), dtype=np.uint32)
+    assert L.lgpu_film_write(f.h, up.ctypes.data_as(C.c_void_p), cnt.ctypes.data_as(C.c_void_p)) == abi.OK
+    assert L.lgpu_film_read(f.h, down.ctypes.data_as(C.c_void_p), None) == abi.OK
+    np.testing.assert_array_equal(down, up)
+    np.testing.assert_array_equal(f.read()[0].reshape(-1), up)
+    f.close()
+    L.hipHostFree(p)

@@ -69,3 +69,30 @@ def test_noalloc_rejects_capacity_beyond_scratch(dev):
     del keep
     f.close()
     s.close()
+
+
+@pytest.mark.parametrize("integrator", [abi.INTEGRATOR_VOLPATH, abi.INTEGRATOR_MIS_VOLPATH])
+@pytest.mark.parametrize("name", ["fog", "grid", "points"])
+def test_noalloc_volumetric_matches_render(dev, integrator, name):
+    """The volumetric stage (light lookups, shading and visibility rays in kernels of their own) outside the
+    pipelined loop: a scene whose lights a sampled direction reaches, a grid, and point lights only."""
+    sd = {"fog": scene.fog_cornell, "grid": lambda: scene.fog_cornell("grid"), "points": lambda: scene.media_scene(res=8, n_points=3)}[name]()
+    s = gpu.Scene(dev)
+    keep = sd.push(s, abi.LIGHTS_TREE)
+    for W, H, spp in ((160, 120, 10), (24, 17, 3)):  # 192,000 paths (several pool waves), then fewer
+        cam = (scene.media_camera if name == "points" else scene.cornell_camera)(W, H)
+        fa, fb = gpu.Film(dev, W, H), gpu.Film(dev, W, H)
+        kw = dict(max_bounces=8, min_bounces=3, spectral=abi.SPECTRAL_HERO4, estimator=abi.ESTIMATOR_CORRECTED,
+                  integrator=integrator)
+        a = gpu.render(gpu.render_desc(s, fa, cam, 0, spp, **kw))
+        rc, b = _noalloc(gpu.render_desc(s, fb, cam, 0, spp, **kw))
+        assert rc == abi.OK, gpu.lib().lgpu_last_error()
+        assert b.samples == W * H * spp and b.extension_rays == a.extension_rays
+        sa, ca = fa.read()
+        sb, cb = fb.read()
+        assert np.array_equal(ca, cb) and (ca == spp).all()
+        assert np.array_equal(sa, sb) and (sa != 0).mean() > 0.2
+        fa.close()
+        fb.close()
+    del keep
+    s.close()
