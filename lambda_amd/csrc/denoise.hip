@@ -54,17 +54,20 @@ __device__ inline float Dist2(float4 a, float4 b) {
 
 // One A-Trous pass; taps outside the image are skipped (the weights renormalise). A thread takes kRows
 // pixels of a column, `step` rows apart: their taps fall on the same kRows + 4 rows, so a tap is loaded
-// once for all of them: 30 loads a pixel instead of 75. A pass over 1920 x 1080 with both guides: 232 us
-// with a tap loaded per pixel, 87 us so (its arithmetic alone is about 65 us).
+// once for all of them: 45 loads a pixel with two rows instead of 75. Bound by the latency of those loads,
+// the more so the fewer waves the image gives: the five taps of a row are loaded together (outside the
+// image from its edge, unused). Denoise call of five passes with both guides, against one pixel a thread and
+// one load at a time: 1920 x 1080 1.95 -> 0.47 ms, 640 x 480 340 -> 119 us, 135 x 95 120 -> 58 us; with four
+// rows and one load at a time 1080p took 0.50 ms, but 135 x 95 215 us.
 // Taps reach each pixel in row-major order, whatever kRows is. kFilm: the last pass writes the film
 // (sums with counts of 1, the albedo multiplied back).
-constexpr int kRows = 4;
-template <bool kFilm>
+template <int kRows, bool kFilm>
 __global__ void __launch_bounds__(256) k_dn_atrous(const float4 *__restrict__ cin, const float4 *__restrict__ alb,
                                                    const float4 *__restrict__ nrm, AtrousParams p, float4 *__restrict__ cout,
                                                    double *__restrict__ sum, uint32_t *__restrict__ count) {
   const int s = (int)p.step, w = (int)p.w, h = (int)p.h;
-  const int x = blockIdx.x * 64 + threadIdx.x % 64, group = blockIdx.y * 4 + threadIdx.x / 64;
+  const uint32_t across = (p.w + 63) / 64;  // blocks: 64 columns by 4 row groups, row by row
+  const int x = blockIdx.x % across * 64 + threadIdx.x % 64, group = blockIdx.x / across * 4 + threadIdx.x / 64;
   const int y0 = (group / s) * (kRows * s) + group % s;  // rows y0, y0 + s, ...
   if (x >= w || y0 >= h) return;
   float4 cp[kRows], np[kRows], ap[kRows];
@@ -81,25 +84,30 @@ __global__ void __launch_bounds__(256) k_dn_atrous(const float4 *__restrict__ ci
   for (int r = -2; r < kRows + 2; ++r) {
     const int qy = y0 + r * s;
     if (qy < 0 || qy >= h) continue;
-#pragma unroll 1
+    float4 cq[5], nq[5], aq[5];
+#pragma unroll
+    for (int dx = -2; dx <= 2; ++dx) {
+      const size_t qi = (size_t)qy * w + min(max(x + dx * s, 0), w - 1);
+      cq[dx + 2] = cin[qi];
+      nq[dx + 2] = p.hasN ? nrm[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
+      aq[dx + 2] = p.hasA ? alb[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
     for (int dx = -2; dx <= 2; ++dx) {
       const int qx = x + dx * s;
       if (qx < 0 || qx >= w) continue;
       const float kx = dx == 0 ? 0.375f : (dx == 1 || dx == -1 ? 0.25f : 0.0625f);
-      const size_t qi = (size_t)qy * w + qx;
-      const float4 cq = cin[qi];
-      const float4 nq = p.hasN ? nrm[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
-      const float4 aq = p.hasA ? alb[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 c = cq[dx + 2];
 #pragma unroll
       for (int k = 0; k < kRows; ++k) {
         const int dy = r - k;
         if (dy < -2 || dy > 2) continue;
         const float ky = dy == 0 ? 0.375f : (dy == 1 || dy == -1 ? 0.25f : 0.0625f);
-        float e = Dist2(cq, cp[k]) * p.invSc2;
-        if (p.hasN) e += Dist2(nq, np[k]) * p.invSn2;
-        if (p.hasA) e += Dist2(aq, ap[k]) * p.invSa2;
+        float e = Dist2(c, cp[k]) * p.invSc2;
+        if (p.hasN) e += Dist2(nq[dx + 2], np[k]) * p.invSn2;
+        if (p.hasA) e += Dist2(aq[dx + 2], ap[k]) * p.invSa2;
         const float wt = kx * ky * expf(-e);
-        sx[k] += wt * cq.x; sy[k] += wt * cq.y; sz[k] += wt * cq.z; sw[k] += wt;
+        sx[k] += wt * c.x; sy[k] += wt * c.y; sz[k] += wt * c.z; sw[k] += wt;
       }
     }
   }
@@ -118,6 +126,22 @@ __global__ void __launch_bounds__(256) k_dn_atrous(const float4 *__restrict__ ci
       cout[pi] = v;
     }
   }
+}
+
+// Images up to this many pixels take one row a thread, for more waves, larger ones two, for fewer loads:
+// 480 x 270 72 and 82 us, 640 x 480 both 118, 800 x 600 175 and 151, 1920 x 1080 559 and 468.
+constexpr uint32_t kOneRow = 1u << 18;
+
+template <int kRows>
+void LaunchPass(hipStream_t st, const AtrousParams &p, const float4 *src, const float4 *alb, const float4 *nrm, float4 *dst,
+                bool last, lgpu_film out) {
+  const uint64_t span = (uint64_t)kRows * p.step, groups = (p.h + span - 1) / span * p.step;
+  const dim3 g((uint32_t)((p.w + 63) / 64 * ((groups + 3) / 4)));  // one dimension: the second holds 65,535 blocks
+  if (last)
+    hipLaunchKernelGGL((k_dn_atrous<kRows, true>), g, dim3(256), 0, st, src, alb, nrm, p, nullptr, out->sum.as<double>(),
+                       out->count.as<uint32_t>());
+  else
+    hipLaunchKernelGGL((k_dn_atrous<kRows, false>), g, dim3(256), 0, st, src, alb, nrm, p, dst, nullptr, nullptr);
 }
 
 }  // namespace
@@ -165,14 +189,10 @@ lgpu_status lgpu_film_denoise(lgpu_film colour, lgpu_film albedo, lgpu_film norm
     p.hasN = normal ? 1u : 0u;
     p.hasA = albedo ? 1u : 0u;
     p.remod = demod ? 1u : 0u;
-    const uint64_t span = (uint64_t)kRows * p.step, groups = (h + span - 1) / span * p.step;
-    const dim3 g2((w + 63) / 64, (uint32_t)((groups + 3) / 4));
+    const bool last = i + 1 == d->iterations;
     const float4 *a4 = albedo ? ab.as<float4>() : nullptr, *n4 = normal ? nb.as<float4>() : nullptr;
-    if (i + 1 < d->iterations)
-      hipLaunchKernelGGL(k_dn_atrous<false>, g2, dim3(256), 0, st, src, a4, n4, p, dst, nullptr, nullptr);
-    else
-      hipLaunchKernelGGL(k_dn_atrous<true>, g2, dim3(256), 0, st, src, a4, n4, p, nullptr, out->sum.as<double>(),
-                         out->count.as<uint32_t>());
+    if (n <= kOneRow) LaunchPass<1>(st, p, src, a4, n4, dst, last, out);
+    else LaunchPass<2>(st, p, src, a4, n4, dst, last, out);
     std::swap(src, dst);
   }
   const hipError_t le = hipGetLastError();

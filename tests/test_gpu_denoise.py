@@ -100,10 +100,11 @@ def test_denoise_rejects_bad_arguments(dev):
         a.denoise(abi.denoise_desc(), normal=b)
 
 
-@pytest.mark.parametrize("w,h", [(1, 1), (3, 70), (64, 16), (65, 17), (130, 33)])
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 70), (64, 16), (65, 17), (130, 33), (512, 512), (513, 512)])
 @pytest.mark.parametrize("iterations", [1, 3, 6])
 def test_denoise_sizes(dev, w, h, iterations):
-    """Image sizes around the filter's tile (64 columns, 4 rows a step apart), steps up to 32 rows."""
+    """Image sizes around the filter's tile (64 columns, rows a step apart) and on both sides of the size where a
+    thread takes two rows, steps up to 32 rows."""
     rng = np.random.default_rng(w + h)
     films, means = [], []
     for lo, hi in ((0.0, 2.0), (0.1, 0.9), (0.0, 1.0)):
@@ -116,3 +117,16 @@ def test_denoise_sizes(dev, w, h, iterations):
     films[0].denoise(d, albedo=films[1], normal=films[2], out=out)
     c = oracle.denoise(means[0], d, albedo=means[1], normal=means[2])
     np.testing.assert_allclose(_means(out), c, rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("w,h", [(1, 270000), (270000, 1), (1, 530000), (2, 140000)])
+def test_denoise_long_images(dev, w, h):
+    """Images of one or two columns or rows, with more row groups than a grid's second dimension holds blocks:
+    every pixel is filtered (a constant image stays what it is)."""
+    f = gpu.Film(dev, w, h)
+    f.write(np.full((h, w, 3), 0.625))
+    out = gpu.Film(dev, w, h)
+    f.denoise(abi.denoise_desc(iterations=3, sigma_colour=0.9), out=out)
+    np.testing.assert_allclose(_means(out), 0.625, rtol=1e-6)
+    f.close()
+    out.close()
