@@ -47,11 +47,9 @@ lgpu_status lgpu_device_create(int hip_device, lgpu_device *out) {
       return Fail(LGPU_ERR_HIP, "device_create: event creation failed");
     }
   }
-  if (ResolveScratch(d) != LGPU_OK) {
+  if (ResolveScratch(d) != LGPU_OK || InitLoops(d) != LGPU_OK) {
     const std::string msg = lgpu_last_error();
-    for (auto &e : d->ev) (void)hipEventDestroy(e);
-    (void)hipStreamDestroy(d->stream);
-    delete d;
+    (void)lgpu_device_destroy(d);
     return Fail(LGPU_ERR_HIP, msg);
   }
   *out = d;
@@ -70,6 +68,9 @@ lgpu_status lgpu_device_destroy(lgpu_device d) {
     for (void *g : d->guides) d->guide_orphan(g);
   for (auto &e : d->ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto &e : d->pev)
+    if (e) (void)hipEventDestroy(e);
+  if (d->hring) (void)hipHostFree(d->hring);
   if (d->stream) (void)hipStreamDestroy(d->stream);
   delete d;
   return LGPU_OK;

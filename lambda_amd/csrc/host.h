@@ -93,6 +93,14 @@ struct lgpu_device_s {
   void *copier = nullptr;             // pinned buffers and threads of host copies
   void (*copier_free)(void *) = nullptr;
   lgpu::DevBuf work[4];               // temporaries of ray queries and image operations, kept between calls (WorkUse)
+  // Pipelined path loops (render.hip): the bounces' slots on the device, their published copies in pinned
+  // memory (and, behind them, the device clock at a wave's start) and an event per slot, after its bounce.
+  // Made with the device object, so that a render which may not allocate has them too.
+  static constexpr int kSlots = 4;
+  lgpu::DevBuf ring;
+  lgpu::BounceSlot *hring = nullptr;
+  hipEvent_t pev[kSlots] = {};
+  double ms_per_tick = 0.0;           // of the device clock
   void *scratch = nullptr;            // device address of this GPU's no-allocation scratch array
   std::vector<void *> guides;         // live guiding networks (released with the device)
   void (*guide_orphan)(void *) = nullptr;
@@ -152,5 +160,6 @@ struct lgpu_scene_s {
 namespace lgpu {
 lgpu_status CommitScene(lgpu_scene s, uint32_t strategy);
 lgpu_status ResolveScratch(lgpu_device dev);  // render.hip: the no-allocation scratch array's address
+lgpu_status InitLoops(lgpu_device dev);       // render.hip: what the pipelined path loops need
 RenderParams MakeParams(const lgpu_render_desc *d, uint32_t w, uint32_t h);  // render.hip
 }

@@ -825,7 +825,7 @@ bool GuideOnDevice(lgpu_guide g, lgpu_device dev);
 
 struct Wave {
   // two path-state buffers (ping-pong), per-sample radiance, shadow queue
-  DevBuf st[2][9], L, pix, lam, shadow, counters, spill, tcount, scene, ring;
+  DevBuf st[2][9], L, pix, lam, shadow, counters, spill, tcount, scene;
   DevBuf gbins, ghdr;  // guided renders: per path slot, the guide's bin table and {c, sum}
   DevBuf ltot;         // adjoint renders: per path slot, the primal pass's radiance
   DevBuf glist, gcount; // guided renders: the bounce's queue slots that shade a guided vertex
@@ -838,18 +838,6 @@ struct Wave {
   uint32_t *counters_p = nullptr, *spill_p = nullptr;
   unsigned long long *tcount_p = nullptr;
   DevScene *scene_p = nullptr;
-  // pipelined path loop: device slots, their pinned host copies, an event per slot (its bounce is
-  // done), and the device clock at a wave's start (pinned)
-  static constexpr int kSlots = 4;
-  BounceSlot *hring = nullptr;
-  unsigned long long *hwave = nullptr;
-  double ms_per_tick = 0.0;
-  hipEvent_t pev[kSlots] = {};
-  ~Wave() {
-    if (hring) (void)hipHostFree(hring);
-    for (hipEvent_t &e : pev)
-      if (e) (void)hipEventDestroy(e);
-  }
   // Device bytes one path in flight holds (both state buffers, sample state, shadow slot, spill;
   // guided: the bin table and header).
   static uint64_t BytesPerPath(uint32_t spillWords, bool guided = false, bool adjoint = false) {
@@ -873,17 +861,6 @@ struct Wave {
       LGPU_HIP(ghdr.alloc(8ull * n));
       LGPU_HIP(glist.alloc(4ull * n));
       LGPU_HIP(gcount.alloc(256));
-    }
-    if (!hring) {
-      int dev = 0, khz = 0;
-      LGPU_HIP(hipGetDevice(&dev));
-      LGPU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
-      ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
-      LGPU_HIP(ring.alloc(sizeof(BounceSlot) * kSlots));
-      for (hipEvent_t &e : pev)
-        if (!e) LGPU_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-      LGPU_HIP(hipHostMalloc((void **)&hring, sizeof(BounceSlot) * (kSlots + 1), hipHostMallocDefault));
-      hwave = reinterpret_cast<unsigned long long *>(hring + kSlots);
     }
     if (n <= cap) return LGPU_OK;
     cap = 0;  // until every part has grown: a failed growth leaves parts released
@@ -976,8 +953,7 @@ RenderParams MakeParams(const lgpu_render_desc *d, uint32_t w, uint32_t h) {
 }
 
 // Renders `total` paths; list mode when listPix != nullptr (trace_paths). `bound`: a wave already
-// laid out in caller memory (no-allocation entry point): no device or pinned allocation happens and
-// the bounce loop synchronises per bounce instead of running ahead through pinned counter copies.
+// laid out in caller memory (no-allocation entry point): no device or pinned allocation happens.
 // `adj`: adjoint render (image-order waves, volumetric integrator): every wave is traced twice with
 // the same random numbers, the primal pass (film accumulation, per-path radiance kept) and the
 // adjoint replay that scatters the gradients.
@@ -1043,6 +1019,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
   if (countTrav) LGPU_HIP(hipMemsetAsync(W.tcount_p, 0, 40, stream));
   lgpu_guide G = d->guide;
   GuideRefs gref{};
+  unsigned long long *hwave = reinterpret_cast<unsigned long long *>(dev->hring + lgpu_device_s::kSlots);
   // pipelined loops: a bounce's last stage lasts until the next bounce begins. A wave's last one: until the
   // empty bounce issued behind it does (slot `tail`), read before a later wave takes the slot again; neither
   // the empty bounces nor what follows the wave (a guide's training, the film update) are in it.
@@ -1050,13 +1027,13 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
   unsigned long long openAt = 0;
   int tail = 0;
   auto CloseStage = [&](unsigned long long at) {
-    if (open) *open += W.ms_per_tick * (double)(at - openAt);
+    if (open) *open += dev->ms_per_tick * (double)(at - openAt);
     open = nullptr;
   };
   auto CloseTail = [&]() -> hipError_t {
     if (!open) return hipSuccess;
-    const hipError_t e = hipEventSynchronize(W.pev[tail]);
-    if (e == hipSuccess) CloseStage(W.hring[tail].extend);
+    const hipError_t e = hipEventSynchronize(dev->pev[tail]);
+    if (e == hipSuccess) CloseStage(dev->hring[tail].extend);
     return e;
   };
   for (uint64_t base = 0; base < total; base += cap) {
@@ -1074,13 +1051,13 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
     cur = 0;
     // path loops other than the direct and utility passes run ahead of the host (below)
     const bool vol = rp.integrator == LGPU_INTEGRATOR_VOLPATH || rp.integrator == LGPU_INTEGRATOR_MIS_VOLPATH;
-    const bool pipelined = (rp.integrator == LGPU_INTEGRATOR_PATH || vol) && !bound;
-    BounceSlot *ring = pipelined ? W.ring.as<BounceSlot>() : nullptr;
+    const bool pipelined = rp.integrator == LGPU_INTEGRATOR_PATH || vol;
+    BounceSlot *ring = pipelined ? dev->ring.as<BounceSlot>() : nullptr;
     float ms;
     if (!pipelined) LGPU_HIP(hipEventRecord(ev[0], stream));
     hipLaunchKernelGGL(k_camera, dim3(Blocks(n)), dim3(kBlock), 0, stream, rp, W.ps[0], W.ss, n, base,
                        listPix ? listPix + base : nullptr, listSmp ? listSmp + base : nullptr,
-                       pipelined ? &ring[Wave::kSlots - 1].next : nullptr, G ? W.gcount.as<uint32_t>() : nullptr, W.hwave);
+                       pipelined ? &ring[lgpu_device_s::kSlots - 1].next : nullptr, G ? W.gcount.as<uint32_t>() : nullptr, hwave);
     LGPU_HIP(hipGetLastError());
     if (!pipelined) {
       LGPU_HIP(hipEventRecord(ev[1], stream));
@@ -1095,15 +1072,15 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
       // host stays up to kLag bounces ahead, retiring them through the published slots. No host
       // round trip, copy, clear or timed event sits between two kernels.
       constexpr int kLag = 3;
-      static_assert(kLag < Wave::kSlots, "a counter slot is reused only after its bounce retired");
+      static_assert(kLag < lgpu_device_s::kSlots, "a counter slot is reused only after its bounce retired");
       uint32_t ub = n, live = n, issued = 0, retired = 0;
       bool done = false;
       LGPU_HIP(CloseTail());  // the camera stage is queued behind it: the GPU does not wait
       while (!done) {
         if (issued < maxIter && issued - retired < (uint32_t)kLag) {
-          const int sl = (int)(issued % Wave::kSlots), prev = (int)((issued + Wave::kSlots - 1) % Wave::kSlots);
+          const int sl = (int)(issued % lgpu_device_s::kSlots), prev = (int)((issued + lgpu_device_s::kSlots - 1) % lgpu_device_s::kSlots);
           uint32_t *cin = &ring[prev].next;
-          BounceSlot *slot = ring + sl, *host = W.hring + sl;
+          BounceSlot *slot = ring + sl, *host = dev->hring + sl;
           // guided: the extension stage lists the bounce's guided vertices for the inference
           const GuideList gl{W.glist.as<uint32_t>(), W.gcount.as<uint32_t>(), G ? gref.max_depth : 0u};
           if (countTrav && G)
@@ -1134,16 +1111,16 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
                                &slot->shadow, W.spill_p, slot, host, G ? W.gcount.as<uint32_t>() : nullptr);
           }
           LGPU_HIP(hipGetLastError());
-          LGPU_HIP(hipEventRecord(W.pev[sl], stream));
+          LGPU_HIP(hipEventRecord(dev->pev[sl], stream));
           cur ^= 1;
           ++issued;
           continue;
         }
         if (retired == issued) break;  // bounce limit reached without termination
-        const int sl = (int)(retired % Wave::kSlots);
-        LGPU_HIP(hipEventSynchronize(W.pev[sl]));
-        const BounceSlot b = W.hring[sl];
-        if (retired == 0) S.ms_camera += W.ms_per_tick * (double)(b.extend - *W.hwave);
+        const int sl = (int)(retired % lgpu_device_s::kSlots);
+        LGPU_HIP(hipEventSynchronize(dev->pev[sl]));
+        const BounceSlot b = dev->hring[sl];
+        if (retired == 0) S.ms_camera += dev->ms_per_tick * (double)(b.extend - *hwave);
         ++retired;
         const uint32_t c0 = b.next, c1 = b.shadow;
         S.extension_rays += live;
@@ -1151,15 +1128,15 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         S.launches_extend++;
         S.launches_shade++;
         CloseStage(b.extend);
-        S.ms_extend += W.ms_per_tick * (double)((G ? b.infer : b.shade) - b.extend);
-        if (G) S.ms_guide_infer += W.ms_per_tick * (double)(b.shade - b.infer);
+        S.ms_extend += dev->ms_per_tick * (double)((G ? b.infer : b.shade) - b.extend);
+        if (G) S.ms_guide_infer += dev->ms_per_tick * (double)(b.shade - b.infer);
         if (vol && (ap || !rp.corrected)) {  // one kernel, its end stamped by the publishing one
-          S.ms_shade += W.ms_per_tick * (double)(b.shadows - b.shade);
+          S.ms_shade += dev->ms_per_tick * (double)(b.shadows - b.shade);
         } else if (vol) {  // one stage: the light lookups, shading and visibility rays
           open = &S.ms_shade;
           openAt = b.shade;
         } else {
-          S.ms_shade += W.ms_per_tick * (double)(b.shadows - b.shade);
+          S.ms_shade += dev->ms_per_tick * (double)(b.shadows - b.shade);
           if (c1) {
             open = &S.ms_shadow;
             openAt = b.shadows;
@@ -1174,7 +1151,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
       }
       if (!done) return Fail(LGPU_ERR_STATE, "render: path wave did not terminate");
       if (issued == retired) open = nullptr;  // no bounce behind the last one of the limit
-      tail = (int)(retired % Wave::kSlots);
+      tail = (int)(retired % lgpu_device_s::kSlots);
       if (G) {  // close the wave's records, then train on them before the next wave infers
         const auto tg = std::chrono::steady_clock::now();
         uint32_t recs = 0;
@@ -1199,14 +1176,10 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
         LGPU_HIP(hipGetLastError());
         LGPU_HIP(hipEventRecord(ev[3], stream));
         Queues q{W.ps[cur ^ 1], W.shadow_p, W.counters_p};
-        if (rp.integrator == LGPU_INTEGRATOR_PATH)
-          LaunchShade(rp.corrected != 0, progs, nullptr, Blocks(count), stream, dscp, rp, W.ps[cur], W.ss, count, nullptr, q);
-        else if (rp.integrator == LGPU_INTEGRATOR_DIRECT)
+        if (rp.integrator == LGPU_INTEGRATOR_DIRECT)
           LaunchShadeDirect(Blocks(count), stream, dsc, rp, W.ps[cur], W.ss, count, q, W.spill_p);
-        else if (rp.integrator >= LGPU_INTEGRATOR_DEPTH)
-          LaunchShadeUtility(Blocks(count), stream, dsc, rp, W.ps[cur], W.ss, count);
         else
-          LaunchShadeVol(Blocks(count), stream, dsc, dscp, rp, W.ps[cur], W.ss, count, q, W.spill_p, ap);
+          LaunchShadeUtility(Blocks(count), stream, dsc, rp, W.ps[cur], W.ss, count);
         LGPU_HIP(hipGetLastError());
         LGPU_HIP(hipEventRecord(ev[4], stream));
         uint32_t cnt[2];
@@ -1366,6 +1339,17 @@ lgpu_status ResolveScratch(lgpu_device dev) {
   LGPU_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
   if (!p || (reinterpret_cast<uintptr_t>(p) & 255u)) return Fail(LGPU_ERR_HIP, "device_create: scratch array unaligned");
   dev->scratch = p;
+  return LGPU_OK;
+}
+
+// What the pipelined loops of a device object need, made with it (that device current).
+lgpu_status InitLoops(lgpu_device dev) {
+  int khz = 0;
+  LGPU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev->device));
+  dev->ms_per_tick = khz > 0 ? 1.0 / khz : 0.0;
+  LGPU_HIP(dev->ring.alloc(sizeof(BounceSlot) * lgpu_device_s::kSlots));
+  for (hipEvent_t &e : dev->pev) LGPU_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  LGPU_HIP(hipHostMalloc((void **)&dev->hring, sizeof(BounceSlot) * (lgpu_device_s::kSlots + 1), hipHostMallocDefault));
   return LGPU_OK;
 }
 

@@ -117,3 +117,20 @@ H.host_hip_budget(before + 400 * MB)
 s.intersect(rays)
 assert live() - before < 100 * MB
 """)
+
+
+def test_noalloc_renders_allocate_nothing_and_do_not_wait_per_bounce(host_hip):
+    """lgpu_render_noalloc takes no device or pinned memory, the first call included, and its path loops read
+    no counter back (their bounces publish it, as in lgpu_render): its one copy is the scene record's."""
+    host_hip("""
+s = gpu.Scene(dev)
+scene.fog_cornell().push(s, abi.LIGHTS_TREE)
+f = gpu.Film(dev, 64, 48)
+before, pinned = live(), H.host_hip_pinned()
+for integrator in (abi.INTEGRATOR_PATH, abi.INTEGRATOR_VOLPATH, abi.INTEGRATOR_MIS_VOLPATH):
+    d = gpu.render_desc(s, f, scene.cornell_camera(64, 48), 0, 2, estimator=abi.ESTIMATOR_CORRECTED, integrator=integrator)
+    copies()
+    assert gpu.lib().lgpu_render_noalloc(C.byref(d), C.byref(abi.RenderStats())) == 0
+    assert [c[2] for c in copies()] == [1], integrator
+    assert live() == before and H.host_hip_pinned() == pinned
+""")
