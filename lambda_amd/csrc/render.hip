@@ -253,15 +253,6 @@ __global__ void __launch_bounds__(kBlock) k_shadow(DevScene sc, SampleState ss, 
 }
 
 // ---------------------------------------------------------------- shade
-__device__ inline void PushShadow(const Queues &q, const ShadowSpec &sh, uint32_t sid, Spec c) {
-  const uint32_t slot = atomicAdd(&q.counters[1], 1u);
-  ShadowRay r;
-  r.o[0] = sh.o.x; r.o[1] = sh.o.y; r.o[2] = sh.o.z; r.tmax = sh.tmax;
-  r.d[0] = sh.d.x; r.d[1] = sh.d.y; r.d[2] = sh.d.z; r.sid = sid;
-  r.contrib[0] = c.c[0]; r.contrib[1] = c.c[1]; r.contrib[2] = c.c[2]; r.contrib[3] = c.c[3];
-  q.shadow[slot] = r;
-}
-
 // The path shade stage's pushes: the extension ray in registers (ExtPush), the shadow ray staged in
 // LDS, both written after one allocation at the block's end (queue.h).
 __device__ inline void StageShadow(ShadowRay &r, const ShadowSpec &sh, uint32_t sid, Spec c) {
