@@ -207,7 +207,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--workload", default="many-light", choices=["many-light", "media", "cornell", "inverse", "batch"],
                     help="inverse: one differentiable-rendering iteration (forward + path-replay adjoint); "
-                         "batch: 64 uneven scenes in one batched graph render vs one render call each")
+                         "batch: 64 uneven scenes in one batched render vs one render call each")
     ap.add_argument("--integrator", default="", choices=["", "path", "direct", "volpath", "mis_volpath"],
                     help="render the workload with another integrator (default: the workload's own)")
     ap.add_argument("--spectral", default="hero4", choices=["hero4", "rgb"])
@@ -457,7 +457,7 @@ def batch_run(args):
     st = gpu.render_batch([desc(j, 2) for j in jobs], autotune=True)
     batch_s = time.perf_counter() - t1
     value = samples / batch_s / 1e6
-    log("batched: %.3f s (%.1f Msamples/s), %d chunks, %d graph nodes, capture %.0f ms"
+    log("batched: %.3f s (%.1f Msamples/s), %d chunks, %d launches, issued in %.0f ms"
         % (batch_s, value, st.chunks, st.graph_nodes, st.ms_capture))
     line = {"metric": "Msamples/s (64-scene batched render, 1 MI355X)", "value": round(value, 3),
             "unit": "Msamples/s", "n_gpus": 1, "steps": spp, "warmup": 1, "ms_per_step": round(batch_s * 1000 / spp, 3),

@@ -363,9 +363,9 @@ lgpu_status lgpu_render_noalloc(const lgpu_render_desc *desc, lgpu_render_stats 
  * and Render.cpp:11-39, across many scenes): every job (scene, film, camera, spp range) renders
  * from one shared path pool whose segments are sized in proportion to the jobs' paths. Every job's
  * waves (camera, bounce iterations with device-side queue counts, film update) are issued on
- * several independent streams without waiting for the device. Jobs take the path or volumetric path integrators with the corrected
- * estimator and no guide; films must be distinct. Each film equals lgpu_render's for the same job
- * (same per-path radiance; the FP64 sums group samples per chunk, so they agree to rounding). */
+ * several independent streams without waiting for the device. Jobs take the path or volumetric path
+ * integrators with the corrected estimator and no guide; films must be distinct. Each film equals
+ * lgpu_render's for the same job bit for bit: the sums go on sample by sample, whatever the chunks. */
 #define LGPU_BATCH_AUTOTUNE 1u /* time pool capacities from 2^23 up to one chunk x 4, 8, 16 branches on whole-batch trials; cached */
 typedef struct lgpu_batch_options {
   uint32_t path_capacity;  /* paths in flight over all jobs (0: 2^24, or the autotuner's choice) */

@@ -88,7 +88,7 @@ struct lgpu_device_s {
   hipEvent_t ev[8] = {};
   void *wave = nullptr;               // path-state pool of the render loop
   void (*wave_free)(void *) = nullptr;
-  void *batch = nullptr;              // capture streams and events of batched renders
+  void *batch = nullptr;              // streams, events and path pool of batched renders
   void (*batch_free)(void *) = nullptr;
   void *copier = nullptr;             // pinned buffers and threads of host copies
   void (*copier_free)(void *) = nullptr;

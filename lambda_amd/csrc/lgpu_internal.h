@@ -384,7 +384,7 @@ struct RenderParams {
   uint32_t pass_normal_g;
 };
 
-// Batched renders (batch.hip) record the single-render kernels through these (render.hip).
+// Batched renders (batch.hip) launch the single-render kernels through these (render.hip).
 void BatchLaunchInit(hipStream_t s, uint32_t *ctr, uint64_t words, uint32_t n);
 void BatchLaunchTrunc(hipStream_t s, const uint32_t *cnt, unsigned long long *acc);
 void BatchLaunchCamera(hipStream_t s, const RenderParams &rp, const PathState &ps, const SampleState &ss, uint32_t n,

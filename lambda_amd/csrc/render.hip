@@ -1201,7 +1201,7 @@ static lgpu_status RunWaves(const lgpu_render_desc *d, uint32_t w, uint32_t h, u
       }
       if (count > 0) return Fail(LGPU_ERR_STATE, "render: path wave did not terminate");
     }
-    if (rep == 1) break;  // the replay's radiance equals the primal pass's: accumulated once
+    if (rep == 1) break;  // the replay's radiance is the primal pass's, to rounding: accumulated once
     if (adj) LGPU_HIP(hipMemcpyAsync(W.ltot.as<float4>(), W.ss.L, 16ull * n, hipMemcpyDeviceToDevice, stream));
     const uint32_t npx = w * h;
     if (!listPix && !out && npx > 0)

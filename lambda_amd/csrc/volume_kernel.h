@@ -21,8 +21,9 @@ namespace lgpu {
 enum VolMode { kVolSplit, kVolSplitLookup, kVolFaithful, kVolAdjoint };
 
 // The scene record comes through a pointer: a by-value argument whose address reaches out-of-line
-// functions is copied into every lane's scratch. The faithful kernel keeps the by-value record and the
-// default registers it has always been run with.
+// functions is copied into every lane's scratch. The faithful kernel keeps the by-value record, and two
+// waves per SIMD (195 registers, 201 with the shader VM); its paths are sorted and its pushes made per block
+// like the others'.
 template <VolMode kMode>
 using VolScene = std::conditional_t<kMode == kVolFaithful, DevScene, const DevScene *__restrict__>;
 __device__ inline const DevScene &SceneOf(const DevScene &sc) { return sc; }

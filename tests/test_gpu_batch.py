@@ -1,8 +1,8 @@
-"""Batched renders (lgpu_render_batch): many scenes from one path pool, one hipGraph per chunk.
+"""Batched renders (lgpu_render_batch): many scenes from one path pool, the jobs on streams side by side.
 
-Bar: each job's film equals lgpu_render of the same job (per-path radiance is identical, the FP64
-film sums group the samples differently: rtol 1e-9), sample counts exactly, for every pool size
-(one chunk, many chunks), for 1 to 8 graph branches and with the autotuner's choice.
+Bar: each job's film equals lgpu_render of the same job (rtol 1e-9 here; bit for bit in
+test_gpu_film_sums.py), sample counts exactly, for every pool size (one chunk, many chunks), for 1
+to 8 branches and with the autotuner's choice.
 """
 import numpy as np
 import pytest

@@ -2,8 +2,8 @@
 
 The no-allocation entry point keeps its path pool in a fixed 64 MiB device array. Two calls in a
 row, the second on a smaller film, must give the films lgpu_render gives: identical sample
-counts, and FP64 sums equal up to the order of the per-wave additions (the pool holds fewer
-paths, so the frame is split into more waves; every path's radiance is the same).
+counts and sums (the pool holds fewer paths, so the frame is split into more waves; every path's
+radiance is the same, and the film's sums go on sample by sample).
 """
 import ctypes as C
 
