@@ -331,47 +331,54 @@ def main():
         "rays ext %d shadow %d" % (args.steps, dt, value, st.ms_extend, st.ms_shade, st.ms_shadow, st.ms_camera,
                                    st.extension_rays, st.shadow_rays))
 
-    # Rooflines (HIP-event kernel times on the render stream).
+    # Rooflines (stage times by the device clock on the render stream).
     # extend: algorithmic bytes per ray = 64 B per 4-wide node record + 48 B per triangle record
     #   the walk fetches (counting pass) + 32 B ray read + 16 B hit write.
     # shade: algorithmic bytes per path vertex = 2 x 96 B path state (read + write), plus 4 B per
-    #   density-grid voxel visited by the vertex's medium walks.
+    #   density-grid voxel visited by the vertex's medium walks. The volumetric stage is timed as one
+    #   and runs up to three kernels: light lookups (scenes with emissive meshes or a sky), shading and
+    #   visibility rays; its traffic is their sum.
     # traffic: the HBM bytes per unit that FETCH_SIZE / WRITE_SIZE measured for this kernel and
     #   workload (calibrated against a copy kernel), read from the committed counter summary.
     bytes_per_ray = None if nodes4_per_ray is None else 64.0 * nodes4_per_ray + 48.0 * tris4_per_ray + 48.0
     bytes_per_vertex = None if voxels_per_vertex is None else 192.0 + 4.0 * voxels_per_vertex
-    shade_name = {"path": "k_shade", "direct": "k_shade_direct"}.get(cfg["integrator"], "k_shade_vol")
+    shade_kernels = {"path": ["k_shade"], "direct": ["k_shade_direct"]}.get(
+        cfg["integrator"], ["k_shade_vol (faithful)"] if args.estimator == "faithful" else
+        ["k_vol_light", "k_shade_vol", "k_vol_shadow"])
     measured = measured_traffic(args.workload)
     valu = measured_valu_busy(args.workload)
     ext_s = st.ms_extend / 1000.0
     sh_s = st.ms_shade / 1000.0
 
-    def roof(kernel, alg, units, secs, launches, unit):
+    def roof(kernels, alg, units, secs, launches, unit):
+        # the kernels of the stage that this workload's counter summary names (all when it names none)
+        named = [k for k in kernels if k in measured] or kernels
+        kernel = " + ".join(named)
         r = {"bound": "hbm", "achieved": None if alg is None else round(alg * units / secs / 1e9, 1),
              "peak": HBM_PEAK_GBS, "unit": "GB/s", "traffic": None, "kernel": kernel, "launches": launches,
              "avg_launch_ms": round(secs * 1000.0 / max(1, launches), 4),
              "alg_bytes_per_unit": None if alg is None else round(alg, 1), "unit_of_work": unit,
              "units_per_launch": round(units / max(1, launches), 1), "units_per_s": round(units / secs, 1)}
         r["frac"] = None if alg is None else round(r["achieved"] / HBM_PEAK_GBS, 4)
-        m = measured.get(kernel)
-        if m:
-            per = m["read"] + m["write"]
+        if named[0] in measured:
+            read, write = (sum(measured[k][way] for k in named) for way in ("read", "write"))
+            per = read + write
             r["traffic"] = round(per * units / max(1, launches), 1)
-            r["traffic_per_unit"] = {"read": m["read"], "write": m["write"], "source": m["source"]}
+            r["traffic_per_unit"] = {"read": round(read, 1), "write": round(write, 1), "source": measured[named[0]]["source"]}
             r["hbm_achieved_GBps"] = round(per * units / secs / 1e9, 1)
         if r["frac"] is not None and r["frac"] > 1.0:
             # the algorithmic bytes are mostly served by L2 and MALL, so HBM does not bound this
             # kernel: report it as VALU-bound with the measured VALU busy share, and its HBM share
             # from the measured traffic
             r["bound"] = "valu"
-            r["frac"] = valu.get(kernel)
+            r["frac"] = valu.get(named[0])
             r["valu_busy_source"] = "profiles/valu_lds_utilisation.md"
             if "hbm_achieved_GBps" in r:
                 r["hbm_frac"] = round(r["hbm_achieved_GBps"] / HBM_PEAK_GBS, 4)
         return r
 
-    ext = roof("k_extend", bytes_per_ray, st.extension_rays, ext_s, st.launches_extend, "extension ray")
-    shd = roof(shade_name, bytes_per_vertex, st.extension_rays, sh_s, st.launches_shade, "path vertex")
+    ext = roof(["k_extend"], bytes_per_ray, st.extension_rays, ext_s, st.launches_extend, "extension ray")
+    shd = roof(shade_kernels, bytes_per_vertex, st.extension_rays, sh_s, st.launches_shade, "path vertex")
     roofline = dict(shd if st.ms_shade >= st.ms_extend else ext)
     roofline["other_kernels"] = [shd if roofline["kernel"] == "k_extend" else ext]
     if args.workload != "many-light":

@@ -12,14 +12,15 @@
 //      equiangular triple with both medium points' direct light (MIS_VOLPATH);
 //   4. otherwise the surface vertex (NEE + BSDF sample) or a pass-through boundary;
 //   5. Russian roulette, then the continuation is appended to the next queue.
-// Traced inline, all rays of a vertex run under the divergent masks of the shading code (8.5 of 64
+// Traced inline, all rays of a vertex run under the divergent masks of the shading code (9 of 64
 // lanes active in the fog room, measured), at the shading code's occupancy of two waves per SIMD.
 // For the corrected estimator the rays therefore run in kernels of their own: step 1 in k_vol_light
 // before, NEE visibility in k_vol_shadow after k_shade_vol, each with the block's rays gathered into
 // full waves. The faithful estimator and the adjoint replay need a ray's result inside the vertex and
-// trace inline. VALU instructions per wave and bounce in the fog room: 18,900 in one kernel; 2,000 here,
-// 2,100 in k_vol_light and 3,300 in k_vol_shadow. Fog room (301 x 211, 16 spp) 13.8 -> 10.1 ms, media
-// workload (1024 x 1024, 4 spp, 128^3 grid) 21.7 -> 17.3 ms.
+// trace inline, and so do the phase-sampled lookups of MIS_VOLPATH's medium points (kVolSplitLookup, scenes
+// with emissive meshes or a sky). VALU instructions in the fog room, a pass: 2.6e9 in one kernel; 0.29e9
+// here, 0.30e9 in k_vol_light and 0.48e9 in k_vol_shadow, at 28, 20 and 20 lanes. Fog room (301 x 211, 16
+// spp) 13.8 -> 10.1 ms, media workload (1024 x 1024, 4 spp, 128^3 grid) 21.7 -> 17.3 ms.
 #include "volume_kernel.h"
 
 namespace lgpu {

@@ -35,3 +35,19 @@ def test_committed_measurements_parse():
     assert 0 < bench.measured_valu_busy("many-light")["k_extend"] <= 1
     r = bench.measured_time_to_relmse()
     assert r["plain_s"] > 0 and r["guided_s"] > 0 and r["plain_spp"] > r["guided_spp"]
+
+
+def test_committed_measurements_name_kernels_that_exist():
+    """Every kernel that a committed counter summary names is one of the sources', and the media workload's
+    covers both kernels of its volumetric stage."""
+    import glob
+    import re
+    sys.path.insert(0, ROOT)
+    import bench
+    sources = "".join(open(f).read() for f in glob.glob(os.path.join(ROOT, "lambda_amd", "csrc", "*")) if os.path.isfile(f))
+    kernels = set(re.findall(r"\b(k_[a-z0-9_]+)\s*\(", sources))
+    for w in ("many-light", "media"):
+        names = set(bench.measured_traffic(w)) | set(bench.measured_valu_busy(w))
+        assert names and names <= kernels, names - kernels
+    assert {"k_shade_vol", "k_vol_shadow"} <= set(bench.measured_traffic("media"))
+    assert {"k_shade_vol", "k_vol_shadow"} <= set(bench.measured_valu_busy("media"))
