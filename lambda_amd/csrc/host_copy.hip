@@ -23,11 +23,12 @@ constexpr size_t kChunk = 1u << 20;    // bytes per transfer
 constexpr int kCopyThreads = 6;        // the caller and five helpers
 constexpr int kOwn = 2;                // pinned buffers of a thread: one is copied while the other is on the bus
 constexpr int kChunks = kOwn * kCopyThreads;  // 12 MiB per device object
-// Copies up to these sizes are the runtime's: one chunk to the host; below 32 MiB to the device, where the
-// source's pages are there and the runtime copies from them in place (film writes of 2, 8 and 24 MiB: the
-// runtime 94, 310 and 850 us, chunks 117, 415 and 1030; of 30 MiB in a new array 1.35 ms and 1.85; from 32
-// MiB both are the same, 1.4 ms, and at 96 MiB the chunks are ahead, 4.2 and 3.95).
-constexpr size_t kDirectToHost = 1u << 20, kDirectToDevice = (32u << 20) - 1;
+// Copies up to these sizes are the runtime's: one chunk to the host; 28 MiB to the device, where the source's
+// pages are there and the runtime copies from them in place, at best from pages it has met before. Film
+// writes of 2, 8 and 24 MiB: the runtime 97, 309 and 824 us from the same array each time and 97, 379 and
+// 1030 from several in turn, chunks 108, 415 and 1042 either way; of 30 MiB 1.24, 1.28 and 1.29 ms, of 48
+// MiB 2.08, 2.02 and 1.96. A ray batch of 30.5 MiB and its hits: 3.83 ms by the runtime, 3.55 by chunks.
+constexpr size_t kDirectToHost = 1u << 20, kDirectToDevice = 28u << 20;
 
 struct HostCopier {
   uint8_t *pinned = nullptr;
