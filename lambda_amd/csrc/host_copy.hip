@@ -23,12 +23,10 @@ constexpr size_t kChunk = 1u << 20;    // bytes per transfer
 constexpr int kCopyThreads = 6;        // the caller and five helpers
 constexpr int kOwn = 2;                // pinned buffers of a thread: one is copied while the other is on the bus
 constexpr int kChunks = kOwn * kCopyThreads;  // 12 MiB per device object
-// Copies up to these sizes are the runtime's: one chunk to the host; 28 MiB to the device, where the source's
-// pages are there and the runtime copies from them in place, at best from pages it has met before. Film
-// writes of 2, 8 and 24 MiB: the runtime 97, 309 and 824 us from the same array each time and 97, 379 and
-// 1030 from several in turn, chunks 108, 415 and 1042 either way; of 30 MiB 1.24, 1.28 and 1.29 ms, of 48
-// MiB 2.08, 2.02 and 1.96. A ray batch of 30.5 MiB and its hits: 3.83 ms by the runtime, 3.55 by chunks.
-constexpr size_t kDirectToHost = 1u << 20, kDirectToDevice = 28u << 20;
+// Copies up to this size (one chunk) are the runtime's. In place, as it copies larger arrays to the device, it is
+// faster (film writes of 2, 8 and 24 MiB 97, 309 and 824 us, chunks 108, 415 and 1042), but the pages it has
+// locked cost later: one in three first passes on new films of 8 MiB then took 3 to 5 ms instead of 0.6.
+constexpr size_t kDirect = 1u << 20;
 
 struct HostCopier {
   uint8_t *pinned = nullptr;
@@ -167,7 +165,7 @@ bool Pageable(const void *p) {
 
 hipError_t Copy(lgpu_device d, void *host, void *dev, size_t n, bool down) {
   if (!n) return hipSuccess;
-  if (n > (down ? kDirectToHost : kDirectToDevice) && Pageable(host)) {
+  if (n > kDirect && Pageable(host)) {
     if (!d->copier) {
       try {
         d->copier = new HostCopier();

@@ -37,21 +37,6 @@ for w, h in ((256, 300), (512, 341), (1021, 1531)):
 """)
 
 
-def test_uploads_copy_in_place_until_chunks_are_faster(host_hip):
-    """Film writes up to 28 MiB are one copy from the caller's array; larger ones go through the chunks."""
-    host_hip("""
-for w, h, chunked in ((256, 250, False), (1024, 1024, False), (1280, 1024, True), (2048, 1100, True)):
-    f = gpu.Film(dev, w, h)
-    a = np.random.default_rng(2).random((h, w, 3))
-    copies()
-    f.write(a, np.ones((h, w), dtype=np.uint32))
-    up = [c for c in copies() if c[2] == 1 and c[1] > 64]
-    sums = [c for c in up if c[0] == a.ctypes.data and c[1] == a.nbytes]
-    assert len(sums) == (0 if chunked else 1), (w, h, up)
-    assert (f.read()[0] == a).all()
-""")
-
-
 def test_page_locked_and_device_memory_is_copied_directly(host_hip):
     """A page-locked array, or device memory in the place of a host array, takes one copy of the whole
     range, in both directions and from any place inside the allocation; an ordinary array goes by chunks."""
