@@ -302,8 +302,9 @@ __device__ inline void BlockPush(const Queues &q, bool pushE, const ExtPush &e, 
 // kCorrected: the estimator mode (rp.corrected) as a template argument, so each instantiation
 // carries only its own mode's branches.
 // kPrograms: what the scene's sockets need (DevScene::has_programs); without program sockets the kernel
-// is compiled without the shader VM, spills little, and runs best at four waves per SIMD (with the
-// VM's call frames and call-site spills, six).
+// is compiled without the shader VM, spills little, and runs best at four waves per SIMD. With the VM the
+// kernel's own code is held to six waves' registers, and its calls to the interpreter, whose 180 a kernel
+// has to allocate, leave two.
 // Guide table of one path slot: GuideBin / sampling over the 128 bin weights (sum `tot`).
 __device__ inline float GuideBinPdf(const uint8_t *tab, float tot, uint32_t bin) {
   return (float)tab[bin] / (tot * kGuideBinSr);

@@ -134,3 +134,20 @@ for integrator in (abi.INTEGRATOR_PATH, abi.INTEGRATOR_VOLPATH, abi.INTEGRATOR_M
     assert [c[2] for c in copies()] == [1], integrator
     assert live() == before and H.host_hip_pinned() == pinned
 """)
+
+
+def test_device_object_that_cannot_be_made_leaves_nothing(host_hip):
+    host_hip("""
+before, pinned = live(), H.host_hip_pinned()
+H.host_hip_budget(before)
+try:
+    gpu.Device(0)
+    raise SystemExit("made")
+except gpu.LambdaError as e:
+    assert "memory" in str(e), e
+assert live() == before and H.host_hip_pinned() == pinned
+H.host_hip_budget(before + MB)
+d = gpu.Device(0)
+d.close()
+assert live() == before and H.host_hip_pinned() == pinned
+""")
