@@ -1,5 +1,5 @@
 """The volumetric shade stage at the edges of its 256-path blocks: a path's result does not depend on how many
-paths run beside it (bit for bit, whatever the block that takes it), and the paths are the CPU checker's
+paths run beside it (bit for bit, whatever the block that takes it), and the paths are the CPU oracle's
 (1e-4 relative + 1e-6, 99.9 % of paths as in the media parity tests)."""
 import numpy as np
 import pytest
